@@ -36,6 +36,8 @@ HIP_SOURCES = {
     # the fp32 accumulators between registers on every k step of the GEMM
     # loop (60-124 v_accvgpr_mov_b32 per stage); o projection 31.2 -> 25.2 us
     "gemm_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    # the same, for the same reason
+    "gemm_skinny.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "ktimer.cpp": [],
 }
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -18,7 +18,9 @@
 //  unset   the MFMA kernel wherever its shape rules allow (gemm_mfma_fits),
 //  (=mfma) hipBLASLt's first heuristic choice for the call's exact shape
 //          otherwise: no timing, so identical inputs give identical bits in
-//          every context and process.  Measured per shape (us, MFMA plan /
+//          every context and process.  The MFMA kernel is gemm_skinny.hip for
+//          the outputs it serves (short prompts), gemm_mfma.hip for the rest.
+//          Measured per shape (us, MFMA plan /
 //          hipBLASLt's first choice): the MFMA kernel is faster for q/k/v, o
 //          and down at every m from 512 to 2048 and for gate/up at 512;
 //          hipBLASLt by 1-5 % for the gate/up GEMM alone from 1024 rows on,
@@ -139,11 +141,13 @@ void gemm_state_destroy(GemmState *g) {
 
 namespace {
 
-// The MFMA kernel with its plan for the shape; a split plan first makes sure
+// The MFMA kernel for the shape: the short-prompt kernel (gemm_skinny.hip)
+// where it serves, else gemm_mfma.hip with its plan; a split plan first makes sure
 // the state holds room for its partials and tickets (allocated on the stream's
 // first such call, zeroed once; every call leaves the tickets zero).
 hipError_t run_mfma(GemmState &g, const uint16_t *W, int n, int k, const uint16_t *x, int m, void *y, int ldy,
                     bool y_bf16, bool acc, hipStream_t s) {
+    if (gemm_skinny_serves(n, k, m)) return gemm_skinny(W, n, k, x, m, y, ldy, y_bf16, acc, s);
     const GemmPlan p = gemm_mfma_plan(n, k, m);
     if (p.split == 2) {
         const size_t need = gemm_split_bytes(n, m, p);
@@ -278,21 +282,25 @@ hipError_t time_candidates(GemmState &g, hipblasLtMatmulDesc_t desc, const Layou
 }  // namespace
 
 bool gemm_swiglu(GemmState *g, hipStream_t s, const uint16_t *Wg, const uint16_t *Wu, bool separate, int f, int k,
-                 const uint16_t *x, int m, const uint16_t *gu, uint16_t *act, hipError_t &err) {
+                 const uint16_t *x, int m, const uint16_t *gu, uint16_t *act, bool short_too, hipError_t &err) {
     err = hipSuccess;
     if (!g || m < 1 || f < 1) return false;
     // gu (null: any 16-byte aligned buffer) and its up half gu + f: their
     // alignment is all that enters (f % 8 == 0 below)
     const bool gu_al = ((uintptr_t)gu & 15u) == 0;
-    auto mfma_unsplit = [&](const uint16_t *W, int n) {
-        return gemm_mfma_fits(W, n, k, x, m, act, 2 * f) && g->mode == kPlanned && gemm_mfma_plan(n, k, m).split == 1;
-    };
-    const bool unfused_mfma = separate ? mfma_unsplit(Wg, f) && mfma_unsplit(Wu, f)
-                                       : Wu == Wg + (size_t)f * k && mfma_unsplit(Wg, 2 * f);
+    // each unfused GEMM ([f][k] twice, or the one [2 f][k]) on this library's
+    // kernels: `skinny` on the short-prompt kernel, else unsplit
+    const int n = separate ? f : 2 * f;
+    const bool skinny = gemm_skinny_serves(n, k, m);
+    const bool unsplit = gemm_mfma_plan(n, k, m).split == 1;
+    const bool mfma = g->mode == kPlanned && gemm_mfma_fits(Wg, n, k, x, m, act, 2 * f) &&
+                      (separate ? gemm_mfma_fits(Wu, n, k, x, m, act, 2 * f) : Wu == Wg + (size_t)f * k) &&
+                      (unsplit || (skinny && short_too));
     // launch_rows_swiglu_bf16's 16-byte kernel
     const bool rows_x8 = f % 8 == 0 && gu_al && ((uintptr_t)act & 15u) == 0 && (size_t)m * (f / 8) <= (1u << 30);
-    if (!unfused_mfma || !rows_x8 || !gemm_swiglu_fits(Wg, Wu, f, k, x, m, act, f)) return false;
-    err = gemm_swiglu_mfma(Wg, Wu, f, k, x, m, act, f, s, gemm_mfma_plan(2 * f, k, m));
+    if (!mfma || !rows_x8 || !gemm_swiglu_fits(Wg, Wu, f, k, x, m, act, f)) return false;
+    err = skinny ? gemm_skinny_swiglu(Wg, Wu, f, k, x, m, act, f, s)
+                 : gemm_swiglu_mfma(Wg, Wu, f, k, x, m, act, f, s, gemm_mfma_plan(2 * f, k, m));
     return true;
 }
 

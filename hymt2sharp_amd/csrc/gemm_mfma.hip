@@ -550,6 +550,16 @@ GemmPlan gemm_mfma_plan(int n, int k, int m) {
     return GemmPlan{5, 2};  // a short prompt
 }
 
+// The two-way split of 128 x 64 tiles that fills whole rounds (2048 features x
+// 449-512 tokens) keeps its kernel: its result for a shape is pinned to the
+// forced split's, bit for bit (the short-prompt kernel, which adds four parts
+// of k, takes 8.7 against 11.7 us on o there and 20.5 against 24.3 on down).
+bool gemm_skinny_serves(int n, int k, int m) {
+    if (std::getenv("HYMT_HIP_GEMM_TILE") || gemm_skinny_plan(n, k, m) < 0) return false;
+    const GemmPlan p = gemm_mfma_plan(n, k, m);
+    return !(p.tile == 5 && p.split == 2 && tiles_of(5, n, m) * 2 % 256 == 0);
+}
+
 bool gemm_mfma_fits(const uint16_t *W, int n, int k, const uint16_t *x, int m, const void *y, int ldy) {
     auto a16 = [](const void *p) { return ((uintptr_t)p & 15u) == 0; };
     return n > 0 && n % 128 == 0 && k >= 2 * kBK && k % (2 * kBK) == 0 && m > 0 && ldy >= n && ldy % 4 == 0 &&

@@ -1153,7 +1153,7 @@ int hymt_gemm_swiglu(hymt_ctx *c, const hymt_weight *gate, const hymt_weight *up
         // gu: a 16-byte aligned [m][2 f] buffer of the unfused calls (only its
         // alignment enters the choice)
         if (!gemm_swiglu(c->gemm, c->stream, gate->dense, wu, up != nullptr, f, k, (const uint16_t *)x, m, nullptr,
-                         (uint16_t *)act, e))
+                         (uint16_t *)act, false, e))
             return fail(HYMT_E_UNSUPPORTED,
                         "no fused gate/up + SwiGLU with the unfused calls' bits here (the GEMM mode, a k split for "
                         "this prompt length, the shape or a misaligned x / act)");
@@ -1511,7 +1511,7 @@ int hymt_model_prefill(hymt_model *m, const int32_t *tokens, int n, int pos, flo
                 const uint16_t *wg = Ly.w[4]->dense, *wu = Ly.w[5] ? Ly.w[5]->dense : wg + (size_t)F * H;
                 hipError_t fe = hipSuccess;
                 if (!gu32 && gemm_swiglu(c->gemm, c->stream, wg, wu, Ly.w[5] != nullptr, F, H, xn, rows,
-                                         (const uint16_t *)gu, act, fe)) {
+                                         (const uint16_t *)gu, act, true, fe)) {
                     HIP_TRY(fe);
                 } else {
                     if (!Ly.w[5]) {

@@ -96,6 +96,20 @@ size_t gemm_split_bytes(int n, int m, GemmPlan p);
 int gemm_split_tiles(int n, int m, GemmPlan p);
 hipError_t gemm_bf16_mfma(const uint16_t *W, int n, int k, const uint16_t *x, int m, void *y, int ldy, bool y_bf16,
                           bool accumulate, hipStream_t s, GemmPlan p, const GemmSplitWs *ws);
+// The short-prompt GEMM (gemm_skinny.hip): k split in four inside each
+// workgroup, small tiles.  gemm_skinny_plan: the tile for a shape, -1 where it
+// does not apply.  gemm_skinny_serves: whether the MFMA choice takes it: where
+// it applies, no tile is forced (HYMT_HIP_GEMM_TILE) and the shape is not one
+// whose two-way split of 128 x 64 tiles fills whole rounds of the chip.
+// Operands as gemm_mfma_fits (gemm_swiglu_fits); every tile gives the same
+// bits, and gemm_skinny_swiglu those of gemm_skinny's bf16 output followed by
+// launch_rows_swiglu_bf16's 16-byte kernel.
+int gemm_skinny_plan(int n, int k, int m);
+bool gemm_skinny_serves(int n, int k, int m);
+hipError_t gemm_skinny(const uint16_t *W, int n, int k, const uint16_t *x, int m, void *y, int ldy, bool y_bf16,
+                       bool accumulate, hipStream_t s);
+hipError_t gemm_skinny_swiglu(const uint16_t *Wg, const uint16_t *Wu, int f, int k, const uint16_t *x, int m,
+                              uint16_t *act, int ld, hipStream_t s);
 // act[m][f] (rows ld elements apart) = silu(g) u, bf16, with g and u the
 // bf16-rounded products x . Wg^T and x . Wu^T (Wg, Wu: [f][k]): the gate/up
 // GEMM and rows_swiglu_bf16 in one launch of the MFMA kernel, unsplit (plan:
@@ -113,7 +127,10 @@ hipError_t gemm_swiglu_mfma(const uint16_t *Wg, const uint16_t *Wu, int f, int k
 // launch_rows_swiglu_bf16 -- is the MFMA kernel unsplit for every GEMM and the
 // 16-byte row kernel, so that the fused call's bits equal theirs; else returns
 // false having enqueued nothing (the caller issues the unfused calls).
+// With short_too it also serves prompts whose unfused GEMMs split k in the
+// short-prompt kernel (the fused form keeps their bits; hymt_gemm_swiglu
+// refuses those lengths, the model's prefill takes them).
 bool gemm_swiglu(GemmState *g, hipStream_t s, const uint16_t *Wg, const uint16_t *Wu, bool separate, int f, int k,
-                 const uint16_t *x, int m, const uint16_t *gu, uint16_t *act, hipError_t &err);
+                 const uint16_t *x, int m, const uint16_t *gu, uint16_t *act, bool short_too, hipError_t &err);
 
 }  // namespace hymt
