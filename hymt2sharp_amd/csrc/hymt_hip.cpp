@@ -635,6 +635,45 @@ int hymt_attn_decode_noalloc(hymt_ctx *c, int layer, int pos, const float *q, co
     return decode_impl(c, layer, pos, q, k, v, qnw, knw, out, HYMT_FLAG_DEVICE_PTRS, ml, acc);
 }
 
+// The number of work items each block pair's kv range splits into, the same
+// for every pair (1: unsplit), or 0 where the range is cut by a tile count
+// instead (below).  At most 256 / pairs (rounded down), so that the items are
+// one round of the chip: a workgroup holds a CU's LDS, and a few items more
+// than 256 cost a whole second round (1000 rows over 8192: 4 ns 79 us, 2 ns
+// 75 us, unsplit 112 us; 700 rows 89 -> 66 us against a cut that made 264
+// items).  The same count for every pair, because the kernels then find their
+// item in closed form instead of by a loop over the pairs.
+//
+// Up to 304 rows every split shortens the call and the longest is taken;
+// beyond, the partials' round trip weighs against the tiles saved.  Fitted to
+// 310-1020 rows over 0-8192 positions with 1-6 splits: 1.4 us per step of two
+// tiles (64 positions each) and 5 ns per row and split, e.g. 512 rows: over 0
+// 17.5 / 19.3 / 20.5 us for 1 / 2 / 4 splits, over 2048 39.7 / 30.7 / 27.2.
+// Over a short cache (under 48 tiles) up to 304 rows keep the cut by tiles: the
+// two differ there by less than a step.
+static int uniform_splits(int pos, int seq, int nb16, int npairs, int kv_heads, int max_tiles) {
+    const int most = 256 / (npairs * kv_heads);
+    if (most < 1) return 0;
+    int best = 1;
+    if (nb16 <= 19) {
+        if (max_tiles < 48) return 0;
+        const int cap = std::max(4, (max_tiles + most - 1) / most);
+        best = (max_tiles + cap - 1) / cap;
+    } else {
+        const int shortest = pair_tiles(pos, npairs - 1, nb16, seq);
+        long best_cost = -1;
+        for (int ns = 1; ns <= std::min(most, shortest); ns++) {
+            const int steps = ((max_tiles + ns - 1) / ns + 1) / 2;
+            const long cost = 280L * steps + (ns > 1 ? (long)seq * ns : 0);  // units of 5 ns
+            if (best_cost < 0 || cost < best_cost) {
+                best_cost = cost;
+                best = ns;
+            }
+        }
+    }
+    return (max_tiles + best - 1) / best <= kItemTiles ? best : 0;
+}
+
 // q_ld / kv_ld: elements from one q (k, v) row to the next; 0 = packed rows
 // out_bf16 (the model's prefill): out receives bf16 bits, the o-projection
 // GEMM's input, rounded as hymt_to_bf16 rounds the fp32 output
@@ -729,29 +768,33 @@ static int prefill_impl(hymt_ctx *c, int layer, int pos, int seq, const void *q,
             for (int b = 0; b < npages; b++) f.pages[b] = c->pages.phys(b);
             for (int b = npages; b < kArgPages; b++) f.pages[b] = f.pages[npages - 1];
         }
-        // Work items: split the kv range of block pairs only when the (kv
-        // head, pair) combinations fill less than half the GPU.  From half
-        // up, the merge launch and its partials cost more than the idle CUs
-        // (1531 rows, 192 pairs: 38.5 + 20.0 us split against 25 us whole).
+        // Work items: the kv range of block pairs is split when the (kv head,
+        // pair) combinations fill at most half the GPU.
         int max_tiles = 0;
         for (int pr = 0; pr < f.npairs; pr++) max_tiles = std::max(max_tiles, pair_tiles(pos, pr, f.nb16, seq));
-        int cap = max_tiles;
-        const int pairs = f.npairs * c->kv_heads;
-        if (pairs < 128) {
-            const int per = (256 + pairs - 1) / pairs;
-            cap = std::max(4, (max_tiles + per - 1) / per);
-        }
-        cap = std::min(cap, kItemTiles);
-        f.cap = cap;
-        int items = 0, ns0 = -1;
+        const int uniform_ns = uniform_splits(pos, seq, f.nb16, f.npairs, c->kv_heads, max_tiles);
+        int items = 0, ns0 = -1, cap = max_tiles;
         bool split = false, uniform = true;
-        for (int pr = 0; pr < f.npairs; pr++) {
-            const int ns = (pair_tiles(pos, pr, f.nb16, seq) + cap - 1) / cap;
-            items += ns;
-            split |= ns > 1;
-            uniform &= ns0 < 0 || ns == ns0;
-            ns0 = ns;
+        if (uniform_ns > 0) {
+            items = uniform_ns * f.npairs;
+            split = uniform_ns > 1;
+            ns0 = uniform_ns;
+        } else {
+            const int pairs = f.npairs * c->kv_heads;
+            if (pairs < 128) {
+                const int per = (256 + pairs - 1) / pairs;
+                cap = std::max(4, (max_tiles + per - 1) / per);
+            }
+            cap = std::min(cap, kItemTiles);
+            for (int pr = 0; pr < f.npairs; pr++) {
+                const int ns = (pair_tiles(pos, pr, f.nb16, seq) + cap - 1) / cap;
+                items += ns;
+                split |= ns > 1;
+                uniform &= ns0 < 0 || ns == ns0;
+                ns0 = ns;
+            }
         }
+        f.cap = cap;
         f.split_ns = split && uniform ? ns0 : 0;
         f.items_per_kvh = items;
         if (split) {

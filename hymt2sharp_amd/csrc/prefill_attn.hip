@@ -1109,7 +1109,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(FlashArgs a) {
 
 template <typename T> void launch_merge(const FlashArgs &a, dim3 grid, hipStream_t s) {
     // the largest split count of any pair (pair 0 is the longest)
-    const int ns = flash_splits(pair_tiles(a.pos0, 0, a.nb16, a.seq), a.cap);
+    const int ns = a.split_ns > 1 ? a.split_ns : flash_splits(pair_tiles(a.pos0, 0, a.nb16, a.seq), a.cap);
     KernelSpan span("prefill_merge", s, true);
     if (ns <= 8) launch(span, prefill_merge_kernel<T, 8>, grid, dim3(256), 0, s, a);
     else if (ns <= 16) launch(span, prefill_merge_kernel<T, 16>, grid, dim3(256), 0, s, a);
