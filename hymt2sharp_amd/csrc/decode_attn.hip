@@ -220,14 +220,16 @@ template <int NR, bool FULL> struct RowsIn {
 //     half-chunk loads, the same bytes and cache lines.
 //   f32 pages (row-major K, V^T sub-tiles [16w, 16w+16)): the same operands
 //   as fp32, two 16-byte K loads per ks and one 16-byte V load per db.
-template <typename S> struct PageOps {
+//   VS: the wave holds V of 1 / VS of the dims, those from vs * 128 / VS on.
+template <typename S, int VS> struct PageOps {
     static constexpr bool W4 = sizeof(S) == 4;
+    static constexpr int VN = (W4 ? 8 : 4) / VS;
     static constexpr int KL = W4 ? 8 : 4;
     uint4 k[KL];
     // V: f32 pages one 16-byte load per db; 16-bit pages the whole chunks of
     // dims 16 db + c for db of the lane's row parity (grp & 1), 4 x 16 bytes,
     // whose other halves the partner row takes (v_halves)
-    uint4 v[W4 ? 8 : 4];
+    uint4 v[VN];
     __device__ __forceinline__ void load_k(const S *kpool, size_t pb, int wave, int grp, int c) {
         constexpr int D = kHeadDim, SUB = 16;
         if constexpr (W4) {
@@ -244,35 +246,31 @@ template <typename S> struct PageOps {
             for (int ks = 0; ks < 4; ks++) k[ks] = *(const uint4 *)(kp + 512 * ks);
         }
     }
-    __device__ __forceinline__ void load_v(const S *vpool, size_t pb, int wave, int grp, int c) {
+    __device__ __forceinline__ void load_v(const S *vpool, size_t pb, int wave, int grp, int c, int vs) {
         constexpr int D = kHeadDim, SUB = 16;
-        if constexpr (W4) {
-            const S *vp = vpool + pb + (size_t)(wave * D + c) * SUB + 4 * grp;
+        const S *vp = vpool + pb + 256 * VN * vs +
+                      (W4 ? (size_t)(wave * D + c) * SUB + 4 * grp
+                          : (size_t)(2 * wave + (grp >> 1)) * 1024 + 8 * c + 128 * (grp & 1));
 #pragma unroll
-            for (int db = 0; db < 8; db++) v[db] = *(const uint4 *)(vp + 256 * db);
-        } else {
-            const S *vp = vpool + pb + (size_t)(2 * wave + (grp >> 1)) * 1024 + 8 * c + 128 * (grp & 1);
-#pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = *(const uint4 *)(vp + 256 * j);
-        }
+        for (int j = 0; j < VN; j++) v[j] = *(const uint4 *)(vp + 256 * j);
     }
     // 16-bit pages: the P.V B operands (4 positions of dim 16 db + c, the
     // half grp & 1 of its chunk) from the loaded chunks.  Rows 0/1 (and 2/3)
     // of the wave hold the chunks of even / odd db; one permlane16 swap per
     // dword pair hands each row the halves it lacks: afterwards the first
     // operand holds db = 2 j and the second db = 2 j + 1 in every row.
-    __device__ __forceinline__ void v_halves(uint2 (&o)[8]) const {
+    __device__ __forceinline__ void v_halves(uint2 (&o)[2 * VN]) const {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < VN; j++) {
             const auto a = __builtin_amdgcn_permlane16_swap(v[j].x, v[j].z, false, false);
             const auto b = __builtin_amdgcn_permlane16_swap(v[j].y, v[j].w, false, false);
             o[2 * j] = make_uint2(a[0], b[0]);
             o[2 * j + 1] = make_uint2(a[1], b[1]);
         }
     }
-    __device__ __forceinline__ void load(const S *kpool, const S *vpool, size_t pb, int wave, int grp, int c) {
+    __device__ __forceinline__ void load(const S *kpool, const S *vpool, size_t pb, int wave, int grp, int c, int vs) {
         load_k(kpool, pb, wave, grp, c);
-        load_v(vpool, pb, wave, grp, c);
+        load_v(vpool, pb, wave, grp, c, vs);
     }
 };
 
@@ -298,8 +296,15 @@ template <typename S> struct PageOps {
 //   holds only the new token (L = 4097 runs exactly 256 workgroups).
 // PAGES_ARG: page ids come from the kernel arguments, else from the device
 // page table; both are scalar loads issued first.
-template <typename T, int PPW, bool RUNS, bool PAGES_ARG, bool FULL>
-__global__ __launch_bounds__(256) void decode_attn_mfma_kernel(DecodeArgs a) {
+// NG: groups of 4 waves in the workgroup.  NG = 1 is the split form above.
+//   NG > 1 is the one-launch form for short caches (nsplit = 1): group g takes
+//   pages g PPW .. of every run of NG PPW pages, and the groups' partials meet
+//   in the same combine as the waves', so no partial goes to memory and no
+//   second launch merges them.
+// VS: a workgroup forms 1 / VS of the output dims (grid VS x kv heads in place
+//   of splits x kv heads): every one reads K whole and its slice of V.
+template <typename T, int PPW, bool RUNS, bool PAGES_ARG, bool FULL, int NG, int VS>
+__global__ __launch_bounds__(256 * NG) void decode_attn_mfma_kernel(DecodeArgs a) {
     constexpr int D = kHeadDim, G = kGroup, P = kPage, SUB = 16;
     // f32 pages: each K and V operand is split on the fly into bf16 hi + lo
     // (x - hi rounded again) and both parts go through the MFMA, so K and V
@@ -309,14 +314,21 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(DecodeArgs a) {
     using M = DecMfma<Op>;
     using S = typename T::storage;
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int NW = 4 * NG;  // waves
+    constexpr int DV = kHeadDim / VS, DB = 8 / VS;  // V dims of the workgroup, in blocks of 16
+    static_assert(NG > 1 || VS == 1, "the split form takes whole heads");
+    const int tid = threadIdx.x, lane = tid & 63;
+    // wave `wave` (position part, q head) of group wg (0 for NG = 1)
+    const int wg = NG > 1 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;
+    const int wave = NG > 1 ? (tid >> 6) & 3 : tid >> 6;
     const int grp = lane >> 4, c = lane & 15;  // MFMA lane group / row-col index
-    const int split = blockIdx.x, kvh = blockIdx.y;  // grid (nsplit, kv heads)
+    // grid (nsplit, kv heads), or (VS, kv heads)
+    const int split = NG > 1 ? 0 : blockIdx.x, vs = VS > 1 ? blockIdx.x : 0, kvh = blockIdx.y;
 
     __shared__ __attribute__((aligned(16))) uint16_t s_qop[2][G][D];  // hi/lo q of the 4 heads
-    __shared__ __attribute__((aligned(16))) float s_o[4][2][D][G];    // per wave: hi/lo rows
+    __shared__ __attribute__((aligned(16))) float s_o[NW][2][DV][G];   // per wave: hi/lo rows
     __shared__ __attribute__((aligned(16))) float s_xo[D][G];         // the new token
-    __shared__ float s_m[5][G], s_l[5][G];                             // [4]: the new token
+    __shared__ float s_m[NW + 1][G], s_l[NW + 1][G];                   // [NW]: the new token
 
     // ---- 0. the arguments: one batch of scalar loads and one wait ---------
     // Every argument passes through one empty asm as an output.  The compiler
@@ -339,7 +351,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(DecodeArgs a) {
     int pid[4] = {0, 0, 0, 0};
     if constexpr (PAGES_ARG) {
 #pragma unroll
-        for (int p = 0; p < PPW; p++) pid[p] = a.pages[min(split * PPW + p, kArgPages - 1)];
+        for (int p = 0; p < PPW; p++) pid[p] = a.pages[min((split * NG + wg) * PPW + p, kArgPages - 1)];
     }
     // Pointers that vector loads use are inputs only: an asm output would be
     // a pointer of unknown address space, read by flat loads.  The stores at
@@ -355,8 +367,8 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(DecodeArgs a) {
 
     const int newpos = L - 1;                // cached positions [0, newpos)
     const int ncp = (newpos + P - 1) / P;    // cached pages
-    const int page0 = split * ppw;
-    const int page_end = min(page0 + ppw, ncp);
+    const int page0 = NG > 1 ? 0 : split * ppw;  // of the split; the wave's first run starts wg * PPW further
+    const int page_end = NG > 1 ? ncp : min(page0 + ppw, ncp);
     const int plast = max(page_end - 1, page0);
     const bool last = split == nsplit - 1;
     const size_t page_elems = (size_t)P * D;
@@ -380,10 +392,10 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(DecodeArgs a) {
     // list while the stream is in flight
     int phys_new = 0;
     if constexpr (!PAGES_ARG) phys_new = __builtin_amdgcn_readfirstlane(tab[newpos / P]);
-    PageOps<S> pg[PPW];
+    PageOps<S, VS> pg[PPW];
 #pragma unroll
     for (int p = 0; p < PPW; p++)
-        pg[p].load(kpool, vpool, page_base(PAGES_ARG ? pid[p] : tab_page(page0 + p)), wave, grp, c);
+        pg[p].load(kpool, vpool, page_base(PAGES_ARG ? pid[p] : tab_page(page0 + wg * PPW + p)), wave, grp, c, vs);
     if constexpr (PAGES_ARG) {
         phys_new = a.pages[newpos / P];
         asm volatile("" : "+s"(phys_new));
@@ -396,6 +408,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(DecodeArgs a) {
 #pragma unroll
     for (int e = 0; e < 2; e++) {
         const uint32_t pr = split_pair<Op>(qy[e]);
+        if (NG > 1 && wg) break;  // group 0 shares the heads
         s_qop[0][wave][lane + 64 * e] = (uint16_t)pr;
         s_qop[1][wave][lane + 64 * e] = (uint16_t)(pr >> 16);
     }
@@ -407,7 +420,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(DecodeArgs a) {
     // vmcnt retires in order, so stores issued here would hold up every
     // later wait on the K/V stream.
     S knew_st[2] = {}, vnew_st[2] = {};
-    if (last) {
+    if (NG > 1 ? wg == 0 : last) {
         float ky[2];
         kin.finish(0, ky, lane, half, rdim, norm_k != 0, eps, 1.0f);
         knew_st[0] = to_elem<T>(ky[0]);
@@ -421,8 +434,8 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(DecodeArgs a) {
         s_xo[lane][wave] = l * from_elem<T>(vnew_st[0]);
         s_xo[lane + 64][wave] = l * from_elem<T>(vnew_st[1]);
         if (lane == 0) {
-            s_m[4][wave] = m;
-            s_l[4][wave] = l;
+            s_m[NW][wave] = m;
+            s_l[NW][wave] = l;
         }
     }
     __syncthreads();
@@ -440,12 +453,12 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(DecodeArgs a) {
         return W4 ? SUB * wave + 4 * grp + i
                   : 32 * (wave >> 1) + 8 * (wave & 1) + 4 * (grp >> 1) + 16 * (grp & 1) + i;
     };
-    f32x4 acc[8];
+    f32x4 acc[DB];
 #pragma unroll
-    for (int db = 0; db < 8; db++) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int db = 0; db < DB; db++) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = kFloor2, l_run = 0.0f;  // lanes c < 4: head c
 
-    for (int run0 = page0; run0 < page_end; run0 += PPW) {
+    for (int run0 = page0 + wg * PPW; run0 < page_end; run0 += NG * PPW) {
         // scores of the run's pages (positions at or past pos masked out)
         float sc[PPW][4], mt = kFloor2;
 #pragma unroll
@@ -472,10 +485,10 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(DecodeArgs a) {
         }
         // the next run's K while this run's softmax and P.V proceed
         size_t nb[PPW];
-        const bool more = RUNS && run0 + PPW < page_end;
+        const bool more = RUNS && run0 + NG * PPW < page_end;
         if (more) {
 #pragma unroll
-            for (int p = 0; p < PPW; p++) nb[p] = page_base(tab_page(run0 + PPW + p));
+            for (int p = 0; p < PPW; p++) nb[p] = page_base(tab_page(run0 + NG * PPW + p));
 #pragma unroll
             for (int p = 0; p < PPW; p++) pg[p].load_k(kpool, nb[p], wave, grp, c);
         }
@@ -493,12 +506,12 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(DecodeArgs a) {
         ps = xrow32_sum(xrow16_sum(ps));
         l_run = l_run * alpha + ps;
         m_run = mnew;
-        if (run0 != page0) {  // rescale the running sums of earlier runs
+        if (run0 != page0 + wg * PPW) {  // rescale the running sums of earlier runs
             float al[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) al[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(alpha), i));
 #pragma unroll
-            for (int db = 0; db < 8; db++)
+            for (int db = 0; db < DB; db++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) acc[db][i] *= al[i];
         }
@@ -525,40 +538,57 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(DecodeArgs a) {
             if (run0 + p >= page_end) keep[0] = keep[1] = 0u;
             if constexpr (W4) {
 #pragma unroll
-                for (int db = 0; db < 8; db++) {
+                for (int db = 0; db < DB; db++) {
                     uint2 hi, lo;
                     split4(pg[p].v[db], keep, hi, lo);
                     acc[db] = M::pv(pa, hi, acc[db]);
                     acc[db] = M::pv(pa, lo, acc[db]);
                 }
             } else {
-                uint2 vh[8];
+                uint2 vh[DB];
                 pg[p].v_halves(vh);
 #pragma unroll
-                for (int db = 0; db < 8; db++)
+                for (int db = 0; db < DB; db++)
                     acc[db] = M::pv(pa, make_uint2(vh[db].x & keep[0], vh[db].y & keep[1]), acc[db]);
             }
         }
         // the next run's V (splits of more than PPW pages)
         if (more) {
 #pragma unroll
-            for (int p = 0; p < PPW; p++) pg[p].load_v(vpool, nb[p], wave, grp, c);
+            for (int p = 0; p < PPW; p++) pg[p].load_v(vpool, nb[p], wave, grp, c, vs);
         }
     }
 
     // ---- 5. combine the wave partials (and the new token) ------------------
     // rows 0-3 (grp 0, hi) and 4-7 (grp 1, lo) of every dim go to LDS as
     // 16-byte vectors [wave][part][dim][head]; (m, l) of head c from lane c.
+    const int pw = 4 * wg + wave;
     if (grp < 2) {
 #pragma unroll
-        for (int db = 0; db < 8; db++) *(f32x4 *)&s_o[wave][grp][16 * db + c][0] = acc[db];
+        for (int db = 0; db < DB; db++) *(f32x4 *)&s_o[pw][grp][16 * db + c][0] = acc[db];
     }
     if (lane < G) {
-        s_m[wave][lane] = m_run;
-        s_l[wave][lane] = l_run;
+        s_m[pw][lane] = m_run;
+        s_l[pw][lane] = l_run;
     }
     __syncthreads();
-    {
+    if constexpr (NG > 1) {
+        // thread -> dim d of the workgroup's slice, head hh; the output itself
+        if (256 * NG == DV * G || tid < DV * G) {
+            const int d = tid % DV, hh = tid / DV, dg = vs * DV + d;
+            float Mx = s_m[0][hh], Lx = 0.f, O = 0.f;
+#pragma unroll
+            for (int w = 1; w <= NW; w++) Mx = fmaxf(Mx, s_m[w][hh]);
+#pragma unroll
+            for (int w = 0; w <= NW; w++) {
+                const float o = w < NW ? s_o[w][0][d][hh] + s_o[w][1][d][hh] : s_xo[dg][hh];
+                const float sc = exp2f(s_m[w][hh] - Mx);
+                Lx = fmaf(sc, s_l[w][hh], Lx);
+                O = fmaf(sc, o, O);
+            }
+            out_g[(size_t)(kvh * G + hh) * D + dg] = Lx > 0.0f ? O / Lx : 0.0f;
+        }
+    } else {
         const int d = tid & 127, gp = 2 * (tid >> 7);  // thread -> dim d, heads gp, gp+1
         const int nw = last ? 5 : 4;
         float Mx[2], Lx[2] = {0.f, 0.f}, O[2] = {0.f, 0.f};
@@ -602,7 +632,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(DecodeArgs a) {
         }
     }
     // ---- 6. append the new row to the cache ---------------------------------
-    if (last && wave == 0) {
+    if (last && wave == 0 && wg == 0 && vs == 0) {
         const int t = newpos % P;
         S *kp = (S *)kpool + ((size_t)phys_new * Hkv + kvh) * page_elems;
         S *vp = (S *)vpool + ((size_t)phys_new * Hkv + kvh) * page_elems;
@@ -764,8 +794,9 @@ hipError_t decode_scratch(int device, float **part_ml, float **part_acc, int *ma
 
 using DecodeKernel = void (*)(DecodeArgs);
 
-template <typename T, int PPW, bool RUNS, bool ARGS> DecodeKernel pick_full(bool full) {
-    return full ? decode_attn_mfma_kernel<T, PPW, RUNS, ARGS, true> : decode_attn_mfma_kernel<T, PPW, RUNS, ARGS, false>;
+template <typename T, int PPW, bool RUNS, bool ARGS, int NG = 1, int VS = 1> DecodeKernel pick_full(bool full) {
+    return full ? decode_attn_mfma_kernel<T, PPW, RUNS, ARGS, true, NG, VS>
+                : decode_attn_mfma_kernel<T, PPW, RUNS, ARGS, false, NG, VS>;
 }
 // Instances that launch_decode can reach: page lists in the arguments hold at
 // most kArgPages pages, taken one or two per split; splits of more than two
@@ -785,6 +816,25 @@ template <typename T> DecodeKernel pick_mfma(int ppw, bool args, bool full) {
         }
         return pick_full<T, 1, true, false>(full);
     }
+}
+
+// The one-launch form: kOneSlices workgroups per kv head, each over all
+// positions and a slice of V's dims, of kOneGroups x 4 waves.  What bounds it
+// is the rate at which 16 CUs (kv heads x slices) pull K and V, about 0.3 us a
+// 16-bit page; the slices cut a CU's bytes to K and a quarter of V.  us per
+// call inside a recorded step, split form / one launch (f16, bf16 alike):
+// 1-2 pages 6.6 / 4.1, 3 pages 6.6 / 4.4, 4 pages 6.6 / 4.7, 6 pages 6.6 / 5.4,
+// 8 pages 6.6 / 6.2, 10 pages equal.  fp32 pages carry twice the bytes and the
+// operand split: 2 pages 8.0 / 5.8, 3 pages 8.1 / 6.9, 4 pages 8.0 / 8.3.
+// Whole heads per workgroup (no slices) took 0.4-0.9 us more, 16 waves 0.4-0.8
+// us.  One page a group and run up to 3 pages, two from there (256 positions
+// 4.8 / 4.7, 512 6.4 / 6.2).
+constexpr int kOneGroups = 2, kOneSlices = 4;
+bool one_launch(int kv_dtype, int pages) { return pages >= 1 && pages <= (kv_dtype == 0 ? 3 : 8); }
+template <typename T> DecodeKernel pick_one(int pages, bool full) {
+    if constexpr (sizeof(typename T::storage) == 2)
+        if (pages > 3) return pick_full<T, 2, true, true, kOneGroups, kOneSlices>(full);
+    return pick_full<T, 1, true, true, kOneGroups, kOneSlices>(full);
 }
 
 // Pages per split for `pages` cached pages (at most kMaxSplits splits).
@@ -816,6 +866,15 @@ hipError_t launch_decode(int kv_dtype, const DecodeArgs &args, hipStream_t s) {
     if (in_args && a.ppw > 2) return hipErrorInvalidValue;
     const bool full = a.rope_dim == kHeadDim;
     DecodeKernel k;
+    // A short cache in one launch (pick_one): the split form's second launch
+    // and the partials' round trip cost more than the tiles' longer walk.
+    if (in_args && one_launch(kv_dtype, pages)) {
+        a.nsplit = 1;
+        k = kv_dtype == 0 ? pick_one<F32>(pages, full) : kv_dtype == 1 ? pick_one<F16>(pages, full) : pick_one<BF16>(pages, full);
+        KernelSpan span("decode_attn", s, true);
+        launch(span, k, dim3(kOneSlices, a.kv_heads), dim3(256 * kOneGroups), 0, s, a);
+        return hipGetLastError();
+    }
     switch (kv_dtype) {
     case 0: k = pick_mfma<F32>(a.ppw, in_args, full); break;
     case 1: k = pick_mfma<F16>(a.ppw, in_args, full); break;

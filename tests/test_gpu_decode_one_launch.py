@@ -1,0 +1,52 @@
+"""Decode attention over a short cache, which one launch serves: positions at
+the page edges, at the edges between its forms (one or two pages a wave group,
+then the split form with its merge), against the oracle with the bars of
+test_gpu_decode.py; every head and dim slice, the appended row and a cache
+whose pages are not in order."""
+import numpy as np
+import pytest
+
+from hymt2sharp_amd import HipBackend
+from hymt2sharp_amd._native import BF16, F16, F32
+from tests.attn_cases import BASE, D, EPS, HKV, HQ, cache_rows, max_rel, new_token
+from tests.test_gpu_random_sweep import decode_case
+from tests.test_gpu_decode import ulp_close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+@pytest.mark.parametrize("pos", [1, 63, 64, 65, 127, 128, 129, 191, 192, 193, 256, 257, 383, 511, 512, 513, 576])
+def test_short_cache(oracle, hip_available, dtype, pos):
+    got, ref, (kd, vd), (kr, vr) = decode_case(oracle, dtype, pos, "gamma", config=17, salt=pos)
+    assert max_rel(got, ref) <= 1e-3
+    assert ulp_close(kd, kr, dtype) and ulp_close(vd, vr, dtype)
+
+
+@pytest.mark.parametrize("dtype,rope_dim", [(F16, 64), (BF16, 2), (F32, 0)])
+def test_short_cache_partial_rotary(oracle, hip_available, dtype, rope_dim):
+    for pos in (100, 180):
+        got, ref, _, _ = decode_case(oracle, dtype, pos, "gamma", config=17, salt=pos, rope_dim=rope_dim)
+        assert max_rel(got, ref) <= 1e-3
+
+
+@pytest.mark.parametrize("dtype", [F16, F32])
+def test_pages_out_of_order(hip_available, dtype):
+    """The same rows give the same bits whatever physical pages hold them."""
+    outs = []
+    for shuffle in (False, True):
+        kb, vb = cache_rows(17, 160, salt=3)
+        q, k, v, qnw, knw = new_token(17, 3, "gamma")
+        be = HipBackend(0).configure(HQ, HKV, D, D, BASE, EPS).create_cache(1, 640, dtype)
+        try:
+            if shuffle:  # map far blocks first, then give them back: the free list hands out others
+                be.MapRange(0, 640)
+                be.SetCacheLen(64)
+                be.MapRange(320, 64)
+            be.UploadKv(0, 0, 160, kb, vb)
+            pages = [be.page_of(b) for b in range(3)]
+            outs.append((pages, be.DecodeAttention(0, 160, q[0], k[0], v[0], qnw, knw)))
+        finally:
+            be.Dispose()
+    assert outs[0][0] != outs[1][0]
+    assert np.array_equal(outs[0][1], outs[1][1])
