@@ -8,7 +8,8 @@
 // decode GEMV moves 1-15 MB, so the kernel is as much about memory latency as
 // bandwidth: a lane issues the loads of all its units before it touches x.
 //
-// Work split: 256 threads (4 waves).  A row takes a group of LPR lanes (8..64,
+// Work split of every type but Q4_K, which runs on the matrix cores
+// (gemv_q4k_kernel): 256 threads (4 waves).  A row takes a group of LPR lanes (8..64,
 // a power of two); lane j of the group handles units j + LPR k (k < K =
 // UPR / LPR, UPR = cols / 32 units per row), so neighbouring lanes read
 // neighbouring bytes and a row costs one reduction over its group (DPP).  x
@@ -167,66 +168,27 @@ struct UnitQ8_0 {
     }
 };
 
-// Q4_K (Q4K.cs:8-19, 36-61): 144-byte super-blocks as stored.  Unit u is
+// Q4_K (Q4K.cs:8-19, 36-61) in the tiles of weights.hpp, dequantized (the
+// embedding and the dense copies; the GEMV is gemv_q4k_kernel).  Unit u is
 // super-block u/8, sub = u%8 -> g = sub/2, h = sub%2: qs bytes
-// 32 g + 16 h + [0,16), their low nibbles at 64 g + 16 h + i (scale 2 g),
-// high nibbles at 64 g + 32 + 16 h + i (scale 2 g + 1).
+// 32 g + 16 h + [0,16), their low nibbles at 64 g + 16 h + i (sub-block 2 g),
+// high nibbles at 64 g + 32 + 16 h + i (sub-block 2 g + 1).
 struct UnitQ4_K {
-    static constexpr int kMax = 8;  // units in flight per lane
-    static constexpr int kGrid = 1024;  // workgroups the lane split aims for (see launch_t)
-    uint4 hdr, qs;
+    uint4 qs;
+    uint32_t sm, dd;
     __device__ void load(const WeightDev &w, int r, int u) {
-        const uint8_t *b = (const uint8_t *)w.q + ((size_t)r * (w.cols / 256) + (u >> 3)) * 144;
-        hdr = *(const uint4 *)b;
-        qs = *(const uint4 *)(b + 16 + 16 * (u & 7));
-    }
-    // scales and mins of sub-blocks 2 g and 2 g + 1 (GetScaleMin, Q4K.cs:8-19);
-    // scale bytes s[0..11] are hdr.y, hdr.z, hdr.w, byte k of a dword taken by
-    // shift (a run-time index into a register array would go to scratch)
-    __device__ void scales(int g, int (&sc)[2], int (&m)[2]) const {
-        auto byte = [](uint32_t w, int k) { return (int)((w >> (8 * k)) & 0xFFu); };
-#pragma unroll
-        for (int t = 0; t < 2; t++) {
-            const int j = 2 * g + t;
-            if (j < 4) {
-                sc[t] = byte(hdr.y, j) & 63;
-                m[t] = byte(hdr.z, j) & 63;
-            } else {
-                sc[t] = (byte(hdr.w, j - 4) & 0xF) | ((byte(hdr.y, j - 4) >> 6) << 4);
-                m[t] = (byte(hdr.w, j - 4) >> 4) | ((byte(hdr.z, j - 4) >> 6) << 4);
-            }
-        }
-    }
-    __device__ float dot(const WeightDev &, int, int u, const float *x, const float *xs) const {
-        const int g = (u & 7) >> 1, h = (u & 1);
-        const int base = 256 * (u >> 3) + 64 * g + 16 * h;
-        const float d = h2f(hdr.x & 0xFFFF), dmin = h2f(hdr.x >> 16);
-        int sc[2], m[2];
-        scales(g, sc, m);
-        const uint32_t wd[4] = {qs.x, qs.y, qs.z, qs.w};
-        const float4 *xl = (const float4 *)(x + xpad(base)), *xh = (const float4 *)(x + xpad(base + 32));
-        float al = 0.f, ah = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            // the high nibbles in place: bytes 16 q, summed then scaled by
-            // 1/16 (exact, the sum's roundings scale with it)
-            float lo[4], hi[4];
-            bytes4(masked(wd[i], 0x0F0F0F0Fu), lo);
-            bytes4(masked(wd[i], 0xF0F0F0F0u), hi);
-            al = dot4(lo, xl[i], al);
-            ah = dot4(hi, xh[i], ah);
-        }
-        ah *= 0.0625f;
-        const float sl = xs[base / 8] + xs[base / 8 + 1], sh = xs[base / 8 + 4] + xs[base / 8 + 5];
-        return d * (sc[0] * al + sc[1] * ah) - dmin * (m[0] * sl + m[1] * sh);
+        const int sub = u & 7, lane = (sub >> 1) * 16 + (r & 15);
+        const uint8_t *b = (const uint8_t *)w.q + ((size_t)(r >> 4) * (w.cols / 256) + (u >> 3)) * kQ4Tile;
+        qs = *(const uint4 *)(b + 1024 * (sub & 1) + 16 * lane);
+        sm = *(const uint32_t *)(b + kQ4Scales + 16 * (r & 15) + 4 * (sub >> 1));
+        dd = *(const uint32_t *)(b + kQ4D + 4 * (r & 15));
     }
     __device__ void store(int u, float, float *o) const {
         const int g = (u & 7) >> 1, h = (u & 1);
         const int base = 256 * (u >> 3) + 64 * g + 16 * h;
-        const float d = h2f(hdr.x & 0xFFFF), dmin = h2f(hdr.x >> 16);
-        int sc[2], m[2];
-        scales(g, sc, m);
-        const float d1 = d * sc[0], m1 = dmin * m[0], d2 = d * sc[1], m2 = dmin * m[1];
+        const float d = h2f(dd & 0xFFFF), dmin = h2f(dd >> 16);
+        const float d1 = d * (int)(sm & 0xFF), d2 = d * (int)((sm >> 8) & 0xFF);
+        const float m1 = dmin * (int)((sm >> 16) & 0xFF), m2 = dmin * (int)(sm >> 24);
         const uint32_t wd[4] = {qs.x, qs.y, qs.z, qs.w};
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -552,6 +514,255 @@ __global__ __launch_bounds__(256) void embed_kernel(WeightDev w, int row, float 
     }
 }
 
+// ---- Q4_K on the matrix cores --------------------------------------------------
+// y = W x' for Q4_K, in integers.  The VALU form of the other types spends a
+// convert and an fma per weight, the scales' bit fields, and x and its sums
+// staged by every workgroup behind two barriers: on 120818 x 2048 rows 74 us
+// where the bytes take 25.  Here a super-block's 256 products run on
+// v_mfma_i32_16x16x64_i8, exactly:
+//  - the codes enter as they are, bytes of 0..15 (one mask per four weights);
+//  - x' enters as a 31-bit fixed-point number in four signed bytes, x' s =
+//    sum_p d_p 256^p, s the power of two that brings the super-block's largest
+//    |x'| to [2^29, 2^30): at least fp32's 24 bits of every value within 2^-6
+//    of the largest, and 2^-30 of the largest for the rest;
+//  - the A operand's 16 rows are (digit p, sub-block pair g): row 4 p + g holds
+//    digit p of x' in the k range of lane group g and zeros elsewhere, its 16
+//    columns are weight rows.  So a lane (p, c) receives digit p's sums of row
+//    c over the four low-code sub-blocks 2 g and, from the other two MFMAs, the
+//    high-code ones 2 g + 1, and weighs them by the 6-bit scales in integers
+//    (below 2^25 together).
+// The minima take fp32 sums of x' per sub-block (which also carry an infinity
+// or NaN of x' into the result).  What is rounded is fp32 and per super-block;
+// x' itself is off by 2^-31 of the largest value at most, which after 256 of
+// them is below the rounding of a sum that holds the largest.  rms error over
+// 2048 rows, of the rms of y, here and in the VALU form (2048 to 8192
+// columns): normal x 0.7e-7 to 1.1e-7 (0.9e-7 to 1.4e-7), one value per
+// super-block 100 to 30000 times the others 0.8e-7 to 1.0e-7 (1.1e-7 to
+// 1.3e-7), log-normal magnitudes with sigma 3 0.7e-7 to 0.9e-7 (0.9e-7 to
+// 1.1e-7), all x positive 0.5e-7 to 0.7e-7 (0.4e-7).
+//
+// Work split: a workgroup of NW waves takes RT tiles of 16 rows; wave v takes
+// super-blocks [v NSB, (v + 1) NSB) of all of them, whose x' it prepares for
+// itself in LDS, so nothing waits for another wave until the partial sums of a
+// row meet at the end (where the RMSNorm's factor, a scalar of x, is applied
+// too).  Every load is issued before the first use.
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+template <int CTRL> __device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+// over the 4 rows of 16 lanes, every lane receiving the result
+__device__ __forceinline__ float rows_sum(float v) {
+    auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+__device__ __forceinline__ float rows_max(float v) {
+    auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+// Keeps a wave's LDS accesses in program order (the LDS unit serves them so).
+__device__ __forceinline__ void wave_order() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int RT, int NW, int NSB, int MODE>
+__global__ __launch_bounds__(64 * NW) void gemv_q4k_kernel(WeightDev w, const float *__restrict__ xg,
+                                                           float *__restrict__ y, int flags,
+                                                           const float *__restrict__ nw, float eps) {
+    // a wave's super-blocks as digits, [group][digit][64 columns], and zeros
+    __shared__ __attribute__((aligned(16))) uint8_t s_x[NW][NSB + 1][1024];
+    __shared__ float s_p[NW][RT][16];
+    __shared__ float s_ss[NW];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = lane >> 4, c = lane & 15;
+    const bool out_swiglu = flags & kGemvOutSwiGLU;
+    const int F = w.rows >> 1, nsb = NW * NSB, sb0 = wave * NSB;
+
+    // the lane's columns of super-block s: 4 lane + [0, 4)
+    float4 xv[NSB], gv[NSB];
+#pragma unroll
+    for (int s = 0; s < NSB; s++) {
+        xv[s] = ((const float4 *)xg)[(sb0 + s) * 64 + lane];
+        if constexpr (MODE == 1) gv[s] = ((const float4 *)nw)[(sb0 + s) * 64 + lane];
+        if constexpr (MODE == 2) gv[s] = ((const float4 *)(xg + w.cols))[(sb0 + s) * 64 + lane];
+    }
+    // tile i's row of this lane; with SwiGLU the tiles alternate between gate
+    // rows and the same rows of up
+    uint4 q0[RT][NSB], q1[RT][NSB], sm[RT][NSB];
+    uint32_t dd[RT][NSB];
+#pragma unroll
+    for (int i = 0; i < RT; i++) {
+        const int row = min(out_swiglu ? (i & 1) * F + 16 * ((int)(blockIdx.x * RT + i) >> 1) + c
+                                       : 16 * (int)(blockIdx.x * RT + i) + c,
+                            w.rows - 1);
+        const int r = row & 15, li = grp * 16 + r;
+        const uint8_t *b = (const uint8_t *)w.q + ((size_t)(row >> 4) * nsb + sb0) * kQ4Tile;
+#pragma unroll
+        for (int s = 0; s < NSB; s++) {
+            q0[i][s] = *(const uint4 *)(b + s * kQ4Tile + 16 * li);
+            q1[i][s] = *(const uint4 *)(b + s * kQ4Tile + 1024 + 16 * li);
+            sm[i][s] = *(const uint4 *)(b + s * kQ4Tile + kQ4Scales + 16 * r);
+            dd[i][s] = *(const uint32_t *)(b + s * kQ4Tile + kQ4D + 4 * r);
+        }
+    }
+    // nothing moves across: the weight loads stay ahead of the first wait on x
+    __builtin_amdgcn_sched_barrier(0);
+
+    if (lane < 16) *(uint32_t *)(s_x[wave][NSB] + 4 * lane) = 0;
+    float S0[NSB], S1[NSB], wgt[NSB], ss = 0.f;
+#pragma unroll
+    for (int s = 0; s < NSB; s++) {
+        float v[4] = {xv[s].x, xv[s].y, xv[s].z, xv[s].w};
+        const float g[4] = {gv[s].x, gv[s].y, gv[s].z, gv[s].w};
+        if constexpr (MODE == 1) {  // Ops.RmsNorm (Ops.cs:12-90); the factor comes at the end
+            ss += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] *= g[e];
+        }
+        if constexpr (MODE == 2) {  // Ops.SiLUMulRange (Ops.cs:1016-1052)
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = v[e] / (1.f + expf(-v[e])) * g[e];
+        }
+        // sums over the sub-blocks (8 lanes) of this lane group: 2 grp, 2 grp + 1
+        float a = (v[0] + v[1]) + (v[2] + v[3]);
+        a += dpp<0xB1>(a);
+        a += dpp<0x4E>(a);
+        a += dpp<0x141>(a);
+        const float b = dpp<0x128>(a);  // the other 8 lanes of the row
+        S0[s] = (lane & 8) ? b : a;
+        S1[s] = (lane & 8) ? a : b;
+        float mx = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+        mx = fmaxf(mx, dpp<0xB1>(mx));
+        mx = fmaxf(mx, dpp<0x4E>(mx));
+        mx = fmaxf(mx, dpp<0x141>(mx));
+        mx = fmaxf(mx, dpp<0x140>(mx));
+        mx = rows_max(mx);
+        // 2^k with mx 2^k in [2^29, 2^30), both it and its inverse normal
+        const int e = min(max((int)(__float_as_uint(mx) >> 23), 30), 254);
+        const float sc = __uint_as_float((uint32_t)(283 - e) << 23);
+        wgt[s] = __uint_as_float((uint32_t)(e - 29 + 8 * grp) << 23);  // of digit `grp`
+        // four signed digits of each column: with 0x80 added to the lower
+        // three bytes they are the bytes less 0x80
+        uint32_t t[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) t[j] = ((uint32_t)(int)(v[j] * sc) + 0x00808080u) ^ 0x00808080u;
+        // digit p of the 4 columns as one dword
+        const uint32_t a0 = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u), a1 = __builtin_amdgcn_perm(t[1], t[0], 0x07030602u);
+        const uint32_t b0 = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u), b1 = __builtin_amdgcn_perm(t[3], t[2], 0x07030602u);
+        uint32_t *p = (uint32_t *)(s_x[wave][s] + grp * 256 + 4 * (lane & 15));
+        p[0] = __builtin_amdgcn_perm(b0, a0, 0x05040100u);
+        p[16] = __builtin_amdgcn_perm(b0, a0, 0x07060302u);
+        p[32] = __builtin_amdgcn_perm(b1, a1, 0x05040100u);
+        p[48] = __builtin_amdgcn_perm(b1, a1, 0x07060302u);
+    }
+    wave_order();
+    float acc[RT] = {};
+    // row c of the A operand: digit c / 4 in the columns of group c % 4
+    const int zoff = (c & 3) == grp ? grp * 256 + (c >> 2) * 64 : -1;
+#pragma unroll
+    for (int s = 0; s < NSB; s++) {
+        const i32x4 *xp = (const i32x4 *)(zoff < 0 ? s_x[wave][NSB] : s_x[wave][s] + zoff);
+        const i32x4 xa[4] = {xp[0], xp[1], xp[2], xp[3]};  // low codes' columns, high codes'
+#pragma unroll
+        for (int i = 0; i < RT; i++) {
+            const uint4 a = q0[i][s], b = q1[i][s];
+            constexpr uint32_t M = 0x0F0F0F0Fu;
+            const i32x4 l0 = {(int)(a.x & M), (int)(a.y & M), (int)(a.z & M), (int)(a.w & M)};
+            const i32x4 l1 = {(int)(b.x & M), (int)(b.y & M), (int)(b.z & M), (int)(b.w & M)};
+            const i32x4 h0 = {(int)((a.x >> 4) & M), (int)((a.y >> 4) & M), (int)((a.z >> 4) & M), (int)((a.w >> 4) & M)};
+            const i32x4 h1 = {(int)((b.x >> 4) & M), (int)((b.y >> 4) & M), (int)((b.z >> 4) & M), (int)((b.w >> 4) & M)};
+            i32x4 L = {0, 0, 0, 0}, H = {0, 0, 0, 0};
+            L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[0], l0, L, 0, 0, 0);
+            H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[2], h0, H, 0, 0, 0);
+            L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[1], l1, L, 0, 0, 0);
+            H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[3], h1, H, 0, 0, 0);
+            const uint32_t k[4] = {sm[i][s].x, sm[i][s].y, sm[i][s].z, sm[i][s].w};
+            int t = 0;
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+                t += __mul24((int)(k[g] & 0xFFu), L[g]) + __mul24((int)((k[g] >> 8) & 0xFFu), H[g]);
+            const float d = h2f(dd[i][s] & 0xFFFF), dmin = h2f(dd[i][s] >> 16);
+            const uint32_t kg = grp & 2 ? (grp & 1 ? k[3] : k[2]) : (grp & 1 ? k[1] : k[0]);
+            const float m0 = (float)((kg >> 16) & 0xFFu), m1 = (float)(kg >> 24);
+            acc[i] = fmaf(d, (float)t * wgt[s], acc[i]);
+            acc[i] = fmaf(-dmin, fmaf(m0, S0[s], m1 * S1[s]), acc[i]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < RT; i++) {
+        const float r = rows_sum(acc[i]);  // the digits' and the groups' shares of row c
+        if (grp == 0) s_p[wave][i][c] = r;
+    }
+    if constexpr (MODE == 1) {
+        ss = group_sum(ss, 64);
+        if (lane == 0) s_ss[wave] = ss;
+    }
+    __syncthreads();
+    const int outs = out_swiglu ? RT * 8 : RT * 16;
+    if (tid >= outs) return;
+    float rr = 1.f;
+    if constexpr (MODE == 1) {
+        float t = 0.f;
+#pragma unroll
+        for (int v = 0; v < NW; v++) t += s_ss[v];
+        rr = 1.0f / sqrtf(t / (float)w.cols + eps);
+    }
+    auto sum = [&](int i, int r) {
+        float t = 0.f;
+#pragma unroll
+        for (int v = 0; v < NW; v++) t += s_p[v][i][r];
+        return MODE == 1 ? t * rr : t;
+    };
+    const int i = tid >> 4, r = tid & 15;
+    if (out_swiglu) {
+        const int o = 16 * ((int)(blockIdx.x * RT >> 1) + i) + r;
+        if (o >= F) return;
+        const float gt = sum(2 * i, r), up = sum(2 * i + 1, r);
+        y[o] = gt / (1.f + expf(-gt)) * up;  // Ops.SiLUMul (Ops.cs:1016-1052)
+        return;
+    }
+    const int row = 16 * (int)(blockIdx.x * RT + i) + r;
+    if (row >= w.rows) return;
+    const float t = sum(i, r);
+    y[row] = (flags & kGemvAccumulate) ? y[row] + t : t;
+}
+
+// GGUF blocks (fp16 d and dmin, 12 bytes of 6-bit scales and mins, 128 code
+// bytes; rows x cols / 256 of 144 bytes) into the tiles of weights.hpp: a wave
+// per tile, its lane the tile's lane (group g, row c).
+__global__ __launch_bounds__(256) void q4k_tiles_kernel(const uint8_t *__restrict__ blocks, int rows, int nsb, int tiles,
+                                                        uint8_t *__restrict__ out) {
+    const int tile = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    if (tile >= tiles) return;
+    const int row = tile / nsb * 16 + c, sb = tile % nsb;
+    uint4 hdr = make_uint4(0, 0, 0, 0), q0 = hdr, q1 = hdr;
+    if (row < rows) {
+        const uint8_t *b = blocks + ((size_t)row * nsb + sb) * 144;
+        hdr = *(const uint4 *)b;
+        q0 = *(const uint4 *)(b + 16 + 32 * g);
+        q1 = *(const uint4 *)(b + 32 + 32 * g);
+    }
+    uint32_t sm = 0;  // GetScaleMin (Q4K.cs:8-19) of sub-blocks 2 g, 2 g + 1; scale bytes 0-3, 4-7, 8-11 in y, z, w
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int j = 2 * g + h, k = 8 * (j & 3);
+        const uint32_t y = (hdr.y >> k) & 0xFFu, z = (hdr.z >> k) & 0xFFu, w = (hdr.w >> k) & 0xFFu;
+        const uint32_t sc = j < 4 ? y & 63 : (w & 0xF) | ((y >> 6) << 4), m = j < 4 ? z & 63 : (w >> 4) | ((z >> 6) << 4);
+        sm |= sc << (8 * h) | m << (16 + 8 * h);
+    }
+    uint8_t *t = out + (size_t)tile * kQ4Tile;
+    *(uint4 *)(t + 16 * lane) = q0;
+    *(uint4 *)(t + 1024 + 16 * lane) = q1;
+    *(uint32_t *)(t + kQ4Scales + 16 * c + 4 * g) = sm;
+    if (g == 0) *(uint32_t *)(t + kQ4D + 4 * c) = hdr.x;
+}
+
 const char *gemv_span_name(int type) {
     switch (type) {
     case kW_F32: return "gemv_f32";
@@ -564,13 +775,6 @@ const char *gemv_span_name(int type) {
     }
 }
 
-template <typename U, typename = void> struct HasGrid : std::false_type {};
-template <typename U> struct HasGrid<U, std::void_t<decltype(U::kGrid)>> : std::true_type {};
-template <typename Unit> constexpr int unit_grid() {
-    if constexpr (HasGrid<Unit>::value) return Unit::kGrid;
-    else return 512;
-}
-
 template <typename Unit, bool STQ>
 hipError_t launch_t(const WeightDev &w, const float *x, float *y, int flags, const float *nw, float eps,
                     hipStream_t s) {
@@ -578,15 +782,12 @@ hipError_t launch_t(const WeightDev &w, const float *x, float *y, int flags, con
     // a row's units must fit a wave; a thread stages at most 4 x 8 values of x
     if (w.cols % 2048 != 0 || w.cols > 8192 || upr > Unit::kMax * 64) return hipErrorInvalidValue;
     // lanes per row: the fewest (most units in flight per lane, K <= kMax), but
-    // more until the grid has kGrid workgroups (512 unless the unit says
-    // otherwise): the dequantising arithmetic is then spread over more waves.
-    // Measured on the 32-layer decode step: Q4_K at 1024 (gate|up with 1536
-    // workgroups of 2 units a lane) 0.935 -> 0.906 ms against 512; the other
-    // formats' gate|up GEMVs are a little slower at 1024.
+    // more until the grid has 512 workgroups: the dequantising arithmetic is
+    // then spread over more waves (gate|up GEMVs are a little slower at 1024).
     int lpr = 8;
     while (upr / lpr > Unit::kMax) lpr *= 2;
     auto blocks = [&](int l) { return (w.rows + 4 * (64 / l) - 1) / (4 * (64 / l)); };
-    while (lpr < 64 && blocks(lpr) < unit_grid<Unit>()) lpr *= 2;
+    while (lpr < 64 && blocks(lpr) < 512) lpr *= 2;
     const size_t lds = ((size_t)w.cols + w.cols / 16) * 4 + (size_t)w.cols / 8 * 4;
     const dim3 grid(blocks(lpr));
     KernelSpan span(gemv_span_name(w.type), s, true);
@@ -623,6 +824,54 @@ hipError_t launch_t(const WeightDev &w, const float *x, float *y, int flags, con
     go(integral_constant<int, 4>{}, integral_constant<int, 4>{});
     go(integral_constant<int, 4>{}, integral_constant<int, 8>{});
     if (!ok) return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+template <int RT, int NW, int NSB>
+void launch_q4k_mode(const WeightDev &w, const float *x, float *y, int flags, const float *nw, float eps, int grid,
+                     const KernelSpan &span, hipStream_t s) {
+    const dim3 g(grid), b(64 * NW);
+    if (flags & kGemvInRmsNorm) launch(span, gemv_q4k_kernel<RT, NW, NSB, 1>, g, b, 0, s, w, x, y, flags, nw, eps);
+    else if (flags & kGemvInSwiGLU) launch(span, gemv_q4k_kernel<RT, NW, NSB, 2>, g, b, 0, s, w, x, y, flags, nw, eps);
+    else launch(span, gemv_q4k_kernel<RT, NW, NSB, 0>, g, b, 0, s, w, x, y, flags, nw, eps);
+}
+
+// One tile per workgroup (with SwiGLU a gate and an up tile) and k over as many
+// waves as leave each one or two super-blocks, while that is at most 512
+// workgroups; beyond, 8 waves and two tiles that share a preparation of x'
+// (one at 8192 columns, where two would hold 140 registers).  us per call in a
+// recorded chain, W from HBM, the VALU form / here: 3072 x 2048 + norm 3.7 /
+// 3.3, 2048 x 2048 3.35 / 3.05, 12288 x 2048 + norm + SwiGLU 7.4 / 5.9, 2048 x
+// 6144 5.2 / 4.9 (12 waves of two super-blocks; 8 of three 5.0), 2048 x 8192 in
+// 16 waves 5.5, in 8 6.0; with the norm, 8192 x 2048 4.6 (two tiles 4.6), 16384
+// x 2048 9.1 / 6.2 (one tile 6.4), 40000 x 2048 26 / 11.3, 120818 x 2048 74 /
+// 26.5 (one tile 31.4, four 28.1).
+hipError_t launch_q4k(const WeightDev &w, const float *x, float *y, int flags, const float *nw, float eps,
+                      hipStream_t s) {
+    if (w.cols % 2048 != 0 || w.cols > 8192) return hipErrorInvalidValue;
+    const bool glu = flags & kGemvOutSwiGLU;
+    const int tiles = glu ? 2 * ((w.rows / 2 + 15) / 16) : (w.rows + 15) / 16;
+    const bool few = (glu ? tiles / 2 : tiles) <= 512;
+    KernelSpan span(gemv_span_name(w.type), s, true);
+    auto go = [&](auto waves, auto sbs, int rt) {
+        constexpr int NW = decltype(waves)::value, NSB = decltype(sbs)::value;
+        if (rt == 2) launch_q4k_mode<2, NW, NSB>(w, x, y, flags, nw, eps, (tiles + 1) / 2, span, s);
+        else launch_q4k_mode<1, NW, NSB>(w, x, y, flags, nw, eps, tiles, span, s);
+    };
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
+    using I4 = std::integral_constant<int, 4>;
+    using I8 = std::integral_constant<int, 8>;
+    using I12 = std::integral_constant<int, 12>;
+    using I16 = std::integral_constant<int, 16>;
+    const int rt = glu || !few ? 2 : 1;
+    switch (w.cols / 2048) {
+    case 1: go(I8{}, I1{}, rt); break;
+    case 2: few ? go(I16{}, I1{}, rt) : go(I8{}, I2{}, rt); break;
+    case 3: few ? go(I12{}, I2{}, rt) : go(I8{}, I3{}, rt); break;
+    default: few ? go(I16{}, I2{}, rt) : go(I8{}, I4{}, glu ? 2 : 1); break;
+    }
     return hipGetLastError();
 }
 
@@ -668,12 +917,19 @@ hipError_t launch_gemv(const WeightDev &w, const float *x, float *y, int flags, 
     case kW_F32: return launch_t<UnitF32, false>(w, x, y, flags, nw, eps, s);
     case kW_F16: return launch_t<UnitF16, false>(w, x, y, flags, nw, eps, s);
     case kW_Q8_0: return launch_t<UnitQ8_0, false>(w, x, y, flags, nw, eps, s);
-    case kW_Q4_K: return launch_t<UnitQ4_K, false>(w, x, y, flags, nw, eps, s);
+    case kW_Q4_K: return launch_q4k(w, x, y, flags, nw, eps, s);
     case kW_Q6_K: return launch_t<UnitQ6_K, false>(w, x, y, flags, nw, eps, s);
     case kW_Q2_0C: return launch_t<UnitQ2_0C, false>(w, x, y, flags, nw, eps, s);
     case kW_STQ1_0: return launch_t<UnitSTQ1_0, true>(w, x, y, flags, nw, eps, s);
     default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_q4k_tiles(const void *blocks, int rows, int cols, void *tiles, hipStream_t s) {
+    const int nsb = cols / 256, n = (rows + 15) / 16 * nsb;
+    hipLaunchKernelGGL(q4k_tiles_kernel, dim3((n + 3) / 4), dim3(256), 0, s, (const uint8_t *)blocks, rows, nsb, n,
+                       (uint8_t *)tiles);
+    return hipGetLastError();
 }
 
 hipError_t launch_rows(const WeightDev &w, const int *rows, int row0, int n, float *out, hipStream_t s) {

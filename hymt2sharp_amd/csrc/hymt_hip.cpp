@@ -1012,6 +1012,26 @@ struct hymt_weight {
     uint16_t *dense = nullptr;  // bf16 [rows][cols] copy for the prefill GEMMs (hymt_weight_dense)
 };
 
+// A Q4_K matrix into its tiles, through a device buffer of at most 32 MiB that
+// the call owns (a few rows of tiles at a time), on the null stream as the
+// other types' copy.  Rearranged on the host, the 61-row layer's weights
+// (36 MiB) took 7 ms longer to upload.
+static hipError_t upload_q4k(int rows, int cols, const uint8_t *data, uint8_t *mem) {
+    const size_t rb = (size_t)cols / 256 * 144;
+    const int step = (int)std::min<size_t>((32u << 20) / rb / 16 * 16, ((size_t)rows + 15) / 16 * 16);
+    uint8_t *tmp = nullptr;
+    hipError_t e = hipMalloc((void **)&tmp, rb * (size_t)std::min(step, rows));
+    if (e != hipSuccess) return e;
+    for (int r = 0; r < rows && e == hipSuccess; r += std::min(step, rows - r)) {
+        const int n = std::min(step, rows - r);
+        e = hipMemcpy(tmp, data + rb * (size_t)r, rb * (size_t)n, hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hymt::launch_q4k_tiles(tmp, n, cols, mem + hymt::q4k_tile_bytes(r, cols), nullptr);
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    }
+    const hipError_t f = hipFree(tmp);
+    return e != hipSuccess ? e : f;
+}
+
 int hymt_weight_upload(hymt_ctx *c, int type, int rows, int cols, const void *data, size_t bytes,
                        hymt_weight **out) {
     if (int r = check_ctx(c, false, true)) return r;
@@ -1026,25 +1046,31 @@ int hymt_weight_upload(hymt_ctx *c, int type, int rows, int cols, const void *da
     if (bytes != (size_t)rows * (size_t)rb)
         return fail(HYMT_E_ARG, "weight data is " + std::to_string(bytes) + " bytes, expected " +
                                     std::to_string((size_t)rows * (size_t)rb));
+    const bool tiles = type == hymt::kW_Q4_K;  // rearranged on the device; the others on the host
     hymt::PackedWeight pk;
-    if (!hymt::pack_weight(type, rows, cols, (const uint8_t *)data, pk))
+    if (!tiles && !hymt::pack_weight(type, rows, cols, (const uint8_t *)data, pk))
         return fail(HYMT_E_UNSUPPORTED, "weight type " + std::to_string(type) + " is not supported");
+    const size_t size = tiles ? hymt::q4k_tile_bytes(rows, cols) : pk.buf.size();
     hymt_weight *w = new (std::nothrow) hymt_weight();
     if (!w) return fail(HYMT_E_OOM, "host allocation failed");
     (void)hipSetDevice(c->device);
-    hipError_t e = hipMalloc(&w->mem, pk.buf.size());
+    hipError_t e = hipMalloc(&w->mem, size);
     if (e != hipSuccess) {
         delete w;
         return fail(HYMT_E_OOM, std::string("hipMalloc: ") + hipGetErrorString(e));
     }
-    e = hipMemcpy(w->mem, pk.buf.data(), pk.buf.size(), hipMemcpyHostToDevice);
+    if (tiles)
+        e = upload_q4k(rows, cols, (const uint8_t *)data, (uint8_t *)w->mem);
+    else
+        e = hipMemcpy(w->mem, pk.buf.data(), size, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         (void)hipFree(w->mem);
         delete w;
-        return fail(HYMT_E_DEVICE, std::string("hipMemcpy: ") + hipGetErrorString(e));
+        return fail(e == hipErrorOutOfMemory ? HYMT_E_OOM : HYMT_E_DEVICE,
+                    std::string("weight copy: ") + hipGetErrorString(e));
     }
     uint8_t *base = (uint8_t *)w->mem;
-    w->bytes = pk.buf.size();
+    w->bytes = size;
     w->dev.type = type;
     w->dev.rows = rows;
     w->dev.cols = cols;

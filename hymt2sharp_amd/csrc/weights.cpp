@@ -65,7 +65,6 @@ bool pack_weight(int type, int rows, int cols, const uint8_t *src, PackedWeight 
     switch (type) {
     case kW_F32:
     case kW_F16:
-    case kW_Q4_K:
         alloc(R * rb, 0, 0);
         std::memcpy(out.buf.data(), src, R * rb);
         return true;

@@ -6,7 +6,13 @@
 // unit of a row is read with aligned vector loads:
 //   F32, F16   as stored, [rows][cols]
 //   Q8_0       q: int8 [rows][cols]; d: fp32 [rows][cols/32]
-//   Q4_K       q: the 144-byte super-blocks as stored (already 16-byte aligned)
+//   Q4_K       q: tiles of 16 rows (the last one padded with zeros) x one
+//              super-block of 256 columns, kQ4Tile bytes, [row / 16][cols / 256]:
+//              the code bytes as lane (g, c) = 16 g + c of a wave reads them,
+//              bytes 32 g + [0, 16) of row c at 16 lane and 32 g + [16, 32) at
+//              1024 + 16 lane; at kQ4Scales + 16 c + 4 g the scales of
+//              sub-blocks 2 g and 2 g + 1, then their mins, a byte each; at
+//              kQ4D + 4 c the row's fp16 d and dmin
 //   Q6_K       q: 208-byte super-blocks ql[128] qh[64] scales[16]; d: fp32
 //              [rows][cols/256]
 //   Q2_0C      q: the code bytes [rows][cols/4]; d: fp32 [rows][cols/512]
@@ -26,6 +32,9 @@ namespace hymt {
 // GgmlTensorType codes (GgmlTensorType.cs)
 constexpr int kW_F32 = 0, kW_F16 = 1, kW_Q8_0 = 8, kW_Q4_K = 12, kW_Q6_K = 14, kW_Q2_0C = 40, kW_STQ1_0 = 43;
 
+// the tile of a Q4_K matrix
+constexpr int kQ4Scales = 2048, kQ4D = kQ4Scales + 256, kQ4Tile = kQ4D + 64;
+
 struct WeightDev {
     int type, rows, cols;
     const void *q;
@@ -42,7 +51,14 @@ struct PackedWeight {
     std::vector<uint8_t> buf;
     size_t off_q = 0, off_q2 = SIZE_MAX, off_d = SIZE_MAX;
 };
+// All types but Q4_K, whose blocks launch_q4k_tiles rearranges on the device.
 bool pack_weight(int type, int rows, int cols, const uint8_t *src, PackedWeight &out);
+// Bytes of a Q4_K matrix's tiles, and the tiles from its GGUF blocks (both on
+// the device).
+inline size_t q4k_tile_bytes(int rows, int cols) {
+    return (size_t)((rows + 15) / 16) * (cols / 256) * kQ4Tile;
+}
+hipError_t launch_q4k_tiles(const void *blocks, int rows, int cols, void *tiles, hipStream_t s);
 
 // gemv flags (as HYMT_GEMV_* in include/hymt_hip.h)
 constexpr int kGemvAccumulate = 1, kGemvInRmsNorm = 2, kGemvInSwiGLU = 4, kGemvOutSwiGLU = 8;
