@@ -8,8 +8,8 @@
 // decode GEMV moves 1-15 MB, so the kernel is as much about memory latency as
 // bandwidth: a lane issues the loads of all its units before it touches x.
 //
-// Work split of every type but Q4_K, which runs on the matrix cores
-// (gemv_q4k_kernel): 256 threads (4 waves).  A row takes a group of LPR lanes (8..64,
+// Work split of every type but Q4_K and Q6_K, which run on the matrix cores
+// (gemv_kq_kernel): 256 threads (4 waves).  A row takes a group of LPR lanes (8..64,
 // a power of two); lane j of the group handles units j + LPR k (k < K =
 // UPR / LPR, UPR = cols / 32 units per row), so neighbouring lanes read
 // neighbouring bytes and a row costs one reduction over its group (DPP).  x
@@ -169,7 +169,7 @@ struct UnitQ8_0 {
 };
 
 // Q4_K (Q4K.cs:8-19, 36-61) in the tiles of weights.hpp, dequantized (the
-// embedding and the dense copies; the GEMV is gemv_q4k_kernel).  Unit u is
+// embedding and the dense copies; the GEMV is gemv_kq_kernel).  Unit u is
 // super-block u/8, sub = u%8 -> g = sub/2, h = sub%2: qs bytes
 // 32 g + 16 h + [0,16), their low nibbles at 64 g + 16 h + i (sub-block 2 g),
 // high nibbles at 64 g + 32 + 16 h + i (sub-block 2 g + 1).
@@ -204,68 +204,34 @@ struct UnitQ4_K {
     }
 };
 
-// Q6_K (Q6K.cs:37-66): 208-byte super-blocks ql[128] qh[64] sc[16], d fp32
-// [rows][cols/256].  Unit u: super-block u/8, l8 = u%8 -> half n = l8/4,
-// p = l8%4, l = 8 p + i (i < 8): values at 128 n + 32 j + l for j < 4.
+// Q6_K (Q6K.cs:37-66) in the tiles of weights.hpp, dequantized.  Unit u is
+// super-block u/8, sub = u%8 -> g = sub/2: its sub-blocks of 16 values 4 g + m,
+// m = 2 (sub%2) (low nibbles) and the next (high nibbles).
 struct UnitQ6_K {
-    static constexpr int kMax = 8;  // units in flight per lane
-    uint2 a, b, h, sc;
+    uint4 q, hi;
+    uint32_t sc;
     float d;
     __device__ void load(const WeightDev &w, int r, int u) {
-        const size_t sb = (size_t)r * (w.cols / 256) + (u >> 3);
-        const uint8_t *blk = (const uint8_t *)w.q + sb * 208;
-        const int n = (u & 7) >> 2, p = (u & 3);
-        a = *(const uint2 *)(blk + 64 * n + 8 * p);
-        b = *(const uint2 *)(blk + 64 * n + 32 + 8 * p);
-        h = *(const uint2 *)(blk + 128 + 32 * n + 8 * p);
-        sc = *(const uint2 *)(blk + 192 + 8 * n);
-        d = w.d[sb];
-    }
-    __device__ float dot(const WeightDev &, int, int u, const float *x, const float *xs) const {
-        const int n = (u & 7) >> 2, p = (u & 3);
-        const int base = 256 * (u >> 3) + 128 * n + 8 * p;
-        // int8 scale i (0..7) of this half: byte i of sc, by shift
-        auto scale = [&](int i) { return (float)(int8_t)((((i < 4) ? sc.x : sc.y) >> (8 * (i & 3))) & 0xFFu); };
-        float acc[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int hw = 0; hw < 2; hw++) {  // i = 4 hw + [0, 4)
-            const uint32_t A = hw ? a.y : a.x, B = hw ? b.y : b.x, H = hw ? h.y : h.x;
-            const uint32_t q1 = (A & 0x0F0F0F0Fu) | ((H & 0x03030303u) << 4);
-            const uint32_t q2 = (B & 0x0F0F0F0Fu) | (((H >> 2) & 0x03030303u) << 4);
-            const uint32_t q3 = ((A >> 4) & 0x0F0F0F0Fu) | (((H >> 4) & 0x03030303u) << 4);
-            const uint32_t q4 = ((B >> 4) & 0x0F0F0F0Fu) | (((H >> 6) & 0x03030303u) << 4);
-            uint32_t qq[4] = {q1, q2, q3, q4};
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                asm("" : "+v"(qq[j]));  // one v_cvt_f32_ubyteN per code (see masked)
-                float f[4];
-                bytes4(qq[j], f);
-                acc[j] = dot4(f, *(const float4 *)(x + xpad(base + 32 * j + 4 * hw)), acc[j]);
-            }
-        }
-        float a_ = 0.f;
-#pragma unroll
-        for (int j = 0; j < 4; j++) a_ += scale(p / 2 + 2 * j) * (acc[j] - 32.f * xs[(base + 32 * j) / 8]);
-        return d * a_;
+        const int sub = u & 7, lane = (sub >> 1) * 16 + (r & 15);
+        const uint8_t *b = (const uint8_t *)w.q + ((size_t)(r >> 4) * (w.cols / 256) + (u >> 3)) * kQ6Tile;
+        q = *(const uint4 *)(b + 1024 * (sub & 1) + 16 * lane);
+        hi = *(const uint4 *)(b + kQ6Hi + 16 * lane);
+        sc = *(const uint32_t *)(b + kQ6Scales + 16 * (r & 15) + 4 * (sub >> 1));
+        d = h2f(*(const uint16_t *)(b + kQ6D + 2 * (r & 15)));
     }
     __device__ void store(int u, float, float *o) const {
-        const int n = (u & 7) >> 2, p = (u & 3);
-        const int base = 256 * (u >> 3) + 128 * n + 8 * p;
-        auto scale = [&](int i) { return (float)(int8_t)((((i < 4) ? sc.x : sc.y) >> (8 * (i & 3))) & 0xFFu); };
+        const int s16 = 16 * (u & 1);  // bits of sc, 4 (u & 1) bits of the high ones
+        const float d0 = d * (float)(int8_t)(sc >> s16), d1 = d * (float)(int8_t)(sc >> (s16 + 8));
+        const uint32_t lo[4] = {q.x, q.y, q.z, q.w}, h[4] = {hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
-        for (int hw = 0; hw < 2; hw++) {
-            const uint32_t A = hw ? a.y : a.x, B = hw ? b.y : b.x, H = hw ? h.y : h.x;
-            const uint32_t qq[4] = {(A & 0x0F0F0F0Fu) | ((H & 0x03030303u) << 4),
-                                    (B & 0x0F0F0F0Fu) | (((H >> 2) & 0x03030303u) << 4),
-                                    ((A >> 4) & 0x0F0F0F0Fu) | (((H >> 4) & 0x03030303u) << 4),
-                                    ((B >> 4) & 0x0F0F0F0Fu) | (((H >> 6) & 0x03030303u) << 4)};
+        for (int i = 0; i < 4; i++) {
+            const uint32_t t = h[i] << (4 * (u & 1));
+            const uint32_t c0 = (t & 0xC0C0C0C0u) | ((lo[i] << 2) & 0x3C3C3C3Cu);
+            const uint32_t c1 = ((t << 2) & 0xC0C0C0C0u) | ((lo[i] >> 2) & 0x3C3C3C3Cu);
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                float f[4];
-                bytes4(qq[j], f);
-                const float ds = d * scale(p / 2 + 2 * j);
-#pragma unroll
-                for (int e = 0; e < 4; e++) o[base + 32 * j + 4 * hw + e] = ds * (f[e] - 32.f);
+            for (int e = 0; e < 4; e++) {
+                o[32 * u + 4 * i + e] = d0 * (float)((int8_t)(c0 >> (8 * e)) >> 2);
+                o[32 * u + 16 + 4 * i + e] = d1 * (float)((int8_t)(c1 >> (8 * e)) >> 2);
             }
         }
     }
@@ -514,7 +480,7 @@ __global__ __launch_bounds__(256) void embed_kernel(WeightDev w, int row, float 
     }
 }
 
-// ---- Q4_K on the matrix cores --------------------------------------------------
+// ---- Q4_K and Q6_K on the matrix cores -------------------------------------------
 // y = W x' for Q4_K, in integers.  The VALU form of the other types spends a
 // convert and an fma per weight, the scales' bit fields, and x and its sums
 // staged by every workgroup behind two barriers: on 120818 x 2048 rows 74 us
@@ -541,6 +507,16 @@ __global__ __launch_bounds__(256) void embed_kernel(WeightDev w, int row, float 
 // 1.3e-7), log-normal magnitudes with sigma 3 0.7e-7 to 0.9e-7 (0.9e-7 to
 // 1.1e-7), all x positive 0.5e-7 to 0.7e-7 (0.4e-7).
 //
+// Q6_K the same way: the codes enter as signed bytes 4 (q - 32) (the high two
+// bits stored with 32's flipped, so that two masks and an or make four), each
+// MFMA's lane groups hold one 16-value sub-block each, so a lane (p, c) receives
+// digit p's sums of row c over four of them and weighs them by their signed
+// scales (below 2^29 together).  There are no minima: an infinity or NaN of x'
+// makes the digits' weight NaN.  rms error as above: normal
+// x 0.7e-7 to 0.9e-7 (1.5e-7 to 2.0e-7), outliers 0.8e-7 to 0.9e-7 (1.1e-7 to
+// 1.3e-7), log-normal 0.7e-7 to 0.9e-7 (1.3e-7), all positive 0.7e-7 (1.1e-7 to
+// 1.7e-7).
+//
 // Work split: a workgroup of NW waves takes RT tiles of 16 rows; wave v takes
 // super-blocks [v NSB, (v + 1) NSB) of all of them, whose x' it prepares for
 // itself in LDS, so nothing waits for another wave until the partial sums of a
@@ -551,6 +527,9 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 template <int CTRL> __device__ __forceinline__ float dpp(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
 }
+template <int CTRL> __device__ __forceinline__ uint32_t dpp(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, false);
+}
 // over the 4 rows of 16 lanes, every lane receiving the result
 __device__ __forceinline__ float rows_sum(float v) {
     auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -558,11 +537,11 @@ __device__ __forceinline__ float rows_sum(float v) {
     auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
-__device__ __forceinline__ float rows_max(float v) {
-    auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+__device__ __forceinline__ uint32_t rows_max(uint32_t v) {
+    auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = max((uint32_t)a[0], (uint32_t)a[1]);
+    auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return max((uint32_t)b[0], (uint32_t)b[1]);
 }
 // Keeps a wave's LDS accesses in program order (the LDS unit serves them so).
 __device__ __forceinline__ void wave_order() {
@@ -570,10 +549,11 @@ __device__ __forceinline__ void wave_order() {
     __builtin_amdgcn_wave_barrier();
 }
 
-template <int RT, int NW, int NSB, int MODE>
-__global__ __launch_bounds__(64 * NW) void gemv_q4k_kernel(WeightDev w, const float *__restrict__ xg,
-                                                           float *__restrict__ y, int flags,
-                                                           const float *__restrict__ nw, float eps) {
+template <bool Q6, int RT, int NW, int NSB, int MODE>
+__global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const float *__restrict__ xg,
+                                                          float *__restrict__ y, int flags,
+                                                          const float *__restrict__ nw, float eps) {
+    constexpr int kTile = Q6 ? kQ6Tile : kQ4Tile;
     // a wave's super-blocks as digits, [group][digit][64 columns], and zeros
     __shared__ __attribute__((aligned(16))) uint8_t s_x[NW][NSB + 1][1024];
     __shared__ float s_p[NW][RT][16];
@@ -594,7 +574,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_q4k_kernel(WeightDev w, const fl
     }
     // tile i's row of this lane; with SwiGLU the tiles alternate between gate
     // rows and the same rows of up
-    uint4 q0[RT][NSB], q1[RT][NSB], sm[RT][NSB];
+    uint4 q0[RT][NSB], q1[RT][NSB], qh[RT][NSB], sm[RT][NSB];
     uint32_t dd[RT][NSB];
 #pragma unroll
     for (int i = 0; i < RT; i++) {
@@ -602,13 +582,19 @@ __global__ __launch_bounds__(64 * NW) void gemv_q4k_kernel(WeightDev w, const fl
                                        : 16 * (int)(blockIdx.x * RT + i) + c,
                             w.rows - 1);
         const int r = row & 15, li = grp * 16 + r;
-        const uint8_t *b = (const uint8_t *)w.q + ((size_t)(row >> 4) * nsb + sb0) * kQ4Tile;
+        const uint8_t *b = (const uint8_t *)w.q + ((size_t)(row >> 4) * nsb + sb0) * kTile;
 #pragma unroll
         for (int s = 0; s < NSB; s++) {
-            q0[i][s] = *(const uint4 *)(b + s * kQ4Tile + 16 * li);
-            q1[i][s] = *(const uint4 *)(b + s * kQ4Tile + 1024 + 16 * li);
-            sm[i][s] = *(const uint4 *)(b + s * kQ4Tile + kQ4Scales + 16 * r);
-            dd[i][s] = *(const uint32_t *)(b + s * kQ4Tile + kQ4D + 4 * r);
+            q0[i][s] = *(const uint4 *)(b + s * kTile + 16 * li);
+            q1[i][s] = *(const uint4 *)(b + s * kTile + 1024 + 16 * li);
+            if constexpr (Q6) {
+                qh[i][s] = *(const uint4 *)(b + s * kTile + kQ6Hi + 16 * li);
+                sm[i][s] = *(const uint4 *)(b + s * kTile + kQ6Scales + 16 * r);
+                dd[i][s] = *(const uint16_t *)(b + s * kTile + kQ6D + 2 * r);
+            } else {
+                sm[i][s] = *(const uint4 *)(b + s * kTile + kQ4Scales + 16 * r);
+                dd[i][s] = *(const uint32_t *)(b + s * kTile + kQ4D + 4 * r);
+            }
         }
     }
     // nothing moves across: the weight loads stay ahead of the first wait on x
@@ -629,24 +615,29 @@ __global__ __launch_bounds__(64 * NW) void gemv_q4k_kernel(WeightDev w, const fl
 #pragma unroll
             for (int e = 0; e < 4; e++) v[e] = v[e] / (1.f + expf(-v[e])) * g[e];
         }
-        // sums over the sub-blocks (8 lanes) of this lane group: 2 grp, 2 grp + 1
-        float a = (v[0] + v[1]) + (v[2] + v[3]);
-        a += dpp<0xB1>(a);
-        a += dpp<0x4E>(a);
-        a += dpp<0x141>(a);
-        const float b = dpp<0x128>(a);  // the other 8 lanes of the row
-        S0[s] = (lane & 8) ? b : a;
-        S1[s] = (lane & 8) ? a : b;
-        float mx = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-        mx = fmaxf(mx, dpp<0xB1>(mx));
-        mx = fmaxf(mx, dpp<0x4E>(mx));
-        mx = fmaxf(mx, dpp<0x141>(mx));
-        mx = fmaxf(mx, dpp<0x140>(mx));
+        if constexpr (!Q6) {  // sums over the sub-blocks (8 lanes) of this lane group: 2 grp, 2 grp + 1
+            float a = (v[0] + v[1]) + (v[2] + v[3]);
+            a += dpp<0xB1>(a);
+            a += dpp<0x4E>(a);
+            a += dpp<0x141>(a);
+            const float b = dpp<0x128>(a);  // the other 8 lanes of the row
+            S0[s] = (lane & 8) ? b : a;
+            S1[s] = (lane & 8) ? a : b;
+        }
+        // largest |x'|, as bits (their order is the values', NaN above all)
+        uint32_t mx = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) mx = max(mx, __float_as_uint(v[j]) & 0x7FFFFFFFu);
+        mx = max(mx, dpp<0xB1>(mx));
+        mx = max(mx, dpp<0x4E>(mx));
+        mx = max(mx, dpp<0x141>(mx));
+        mx = max(mx, dpp<0x140>(mx));
         mx = rows_max(mx);
         // 2^k with mx 2^k in [2^29, 2^30), both it and its inverse normal
-        const int e = min(max((int)(__float_as_uint(mx) >> 23), 30), 254);
+        const int e = min(max((int)(mx >> 23), 30), 254);
         const float sc = __uint_as_float((uint32_t)(283 - e) << 23);
         wgt[s] = __uint_as_float((uint32_t)(e - 29 + 8 * grp) << 23);  // of digit `grp`
+        if (Q6 && mx >= 0x7F800000u) wgt[s] = NAN;
         // four signed digits of each column: with 0x80 added to the lower
         // three bytes they are the bytes less 0x80
         uint32_t t[4];
@@ -668,10 +659,30 @@ __global__ __launch_bounds__(64 * NW) void gemv_q4k_kernel(WeightDev w, const fl
 #pragma unroll
     for (int s = 0; s < NSB; s++) {
         const i32x4 *xp = (const i32x4 *)(zoff < 0 ? s_x[wave][NSB] : s_x[wave][s] + zoff);
-        const i32x4 xa[4] = {xp[0], xp[1], xp[2], xp[3]};  // low codes' columns, high codes'
+        const i32x4 xa[4] = {xp[0], xp[1], xp[2], xp[3]};  // Q4_K: low codes' columns, high codes'
 #pragma unroll
         for (int i = 0; i < RT; i++) {
             const uint4 a = q0[i][s], b = q1[i][s];
+            const uint32_t k[4] = {sm[i][s].x, sm[i][s].y, sm[i][s].z, sm[i][s].w};
+            if constexpr (Q6) {
+                const uint32_t h[4] = {qh[i][s].x, qh[i][s].y, qh[i][s].z, qh[i][s].w};
+                const uint32_t lo[2][4] = {{a.x, a.y, a.z, a.w}, {b.x, b.y, b.z, b.w}};
+                int t = 0;
+#pragma unroll
+                for (int m = 0; m < 4; m++) {  // columns 64 g + 16 m + [0, 16): sub-block 4 g + m
+                    i32x4 f;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const uint32_t l = m & 1 ? lo[m >> 1][j] >> 2 : lo[m >> 1][j] << 2;
+                        f[j] = (int)(((h[j] << (2 * m)) & 0xC0C0C0C0u) | (l & 0x3C3C3C3Cu));
+                    }
+                    const i32x4 D = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[m], f, i32x4{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+                    for (int g = 0; g < 4; g++) t += __mul24((int)(int8_t)(k[g] >> (8 * m)), D[g]);
+                }
+                acc[i] = fmaf(h2f(dd[i][s]), (float)t * 0.25f * wgt[s], acc[i]);
+                continue;
+            }
             constexpr uint32_t M = 0x0F0F0F0Fu;
             const i32x4 l0 = {(int)(a.x & M), (int)(a.y & M), (int)(a.z & M), (int)(a.w & M)};
             const i32x4 l1 = {(int)(b.x & M), (int)(b.y & M), (int)(b.z & M), (int)(b.w & M)};
@@ -682,7 +693,6 @@ __global__ __launch_bounds__(64 * NW) void gemv_q4k_kernel(WeightDev w, const fl
             H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[2], h0, H, 0, 0, 0);
             L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[1], l1, L, 0, 0, 0);
             H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[3], h1, H, 0, 0, 0);
-            const uint32_t k[4] = {sm[i][s].x, sm[i][s].y, sm[i][s].z, sm[i][s].w};
             int t = 0;
 #pragma unroll
             for (int g = 0; g < 4; g++)
@@ -763,6 +773,43 @@ __global__ __launch_bounds__(256) void q4k_tiles_kernel(const uint8_t *__restric
     if (g == 0) *(uint32_t *)(t + kQ4D + 4 * c) = hdr.x;
 }
 
+// The same for Q6_K's GGUF blocks (ql 128, qh 64, int8 scales 16, fp16 d: 210
+// bytes, so 2-byte aligned).
+__global__ __launch_bounds__(256) void q6k_tiles_kernel(const uint8_t *__restrict__ blocks, int rows, int nsb, int tiles,
+                                                        uint8_t *__restrict__ out) {
+    const int tile = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    if (tile >= tiles) return;
+    const int row = tile / nsb * 16 + c, sb = tile % nsb;
+    uint32_t q[2][4] = {}, hi[4] = {}, sc = 0, d = 0;
+    if (row < rows) {
+        const uint8_t *b = blocks + ((size_t)row * nsb + sb) * 210;
+        auto rd = [&](int at) {  // 4 bytes, 2-byte aligned
+            return *(const uint16_t *)(b + at) | (uint32_t)*(const uint16_t *)(b + at + 2) << 16;
+        };
+        // columns 64 g + 32 h + [0, 32) are quarter j = 2 (g & 1) + h of half g / 2
+        const int n = g >> 1, nib = 4 * (g & 1);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int j2 = 4 * (g & 1) + 2 * h, at = 64 * n + 32 * h + 4 * i;  // 2 j
+                q[h][i] = ((rd(at) >> nib) & 0x0F0F0F0Fu) | ((rd(at + 16) >> nib) & 0x0F0F0F0Fu) << 4;
+                const uint32_t h0 = (rd(128 + 32 * n + 4 * i) >> j2) & 0x03030303u;
+                const uint32_t h1 = (rd(128 + 32 * n + 16 + 4 * i) >> j2) & 0x03030303u;
+                // bits 7:6 for m = 0 down to 1:0 for m = 3, the upper one (32) flipped
+                hi[i] |= (h0 ^ 0x02020202u) << (6 - 4 * h) | (h1 ^ 0x02020202u) << (4 - 4 * h);
+            }
+        sc = rd(192 + 4 * g);
+        d = *(const uint16_t *)(b + 208);
+    }
+    uint8_t *t = out + (size_t)tile * kQ6Tile;
+    *(uint4 *)(t + 16 * lane) = make_uint4(q[0][0], q[0][1], q[0][2], q[0][3]);
+    *(uint4 *)(t + 1024 + 16 * lane) = make_uint4(q[1][0], q[1][1], q[1][2], q[1][3]);
+    *(uint4 *)(t + kQ6Hi + 16 * lane) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+    *(uint32_t *)(t + kQ6Scales + 16 * c + 4 * g) = sc;
+    if (g == 0) *(uint16_t *)(t + kQ6D + 2 * c) = (uint16_t)d;
+}
+
 const char *gemv_span_name(int type) {
     switch (type) {
     case kW_F32: return "gemv_f32";
@@ -827,13 +874,13 @@ hipError_t launch_t(const WeightDev &w, const float *x, float *y, int flags, con
     return hipGetLastError();
 }
 
-template <int RT, int NW, int NSB>
-void launch_q4k_mode(const WeightDev &w, const float *x, float *y, int flags, const float *nw, float eps, int grid,
-                     const KernelSpan &span, hipStream_t s) {
+template <bool Q6, int RT, int NW, int NSB>
+void launch_kq_mode(const WeightDev &w, const float *x, float *y, int flags, const float *nw, float eps, int grid,
+                    const KernelSpan &span, hipStream_t s) {
     const dim3 g(grid), b(64 * NW);
-    if (flags & kGemvInRmsNorm) launch(span, gemv_q4k_kernel<RT, NW, NSB, 1>, g, b, 0, s, w, x, y, flags, nw, eps);
-    else if (flags & kGemvInSwiGLU) launch(span, gemv_q4k_kernel<RT, NW, NSB, 2>, g, b, 0, s, w, x, y, flags, nw, eps);
-    else launch(span, gemv_q4k_kernel<RT, NW, NSB, 0>, g, b, 0, s, w, x, y, flags, nw, eps);
+    if (flags & kGemvInRmsNorm) launch(span, gemv_kq_kernel<Q6, RT, NW, NSB, 1>, g, b, 0, s, w, x, y, flags, nw, eps);
+    else if (flags & kGemvInSwiGLU) launch(span, gemv_kq_kernel<Q6, RT, NW, NSB, 2>, g, b, 0, s, w, x, y, flags, nw, eps);
+    else launch(span, gemv_kq_kernel<Q6, RT, NW, NSB, 0>, g, b, 0, s, w, x, y, flags, nw, eps);
 }
 
 // One tile per workgroup (with SwiGLU a gate and an up tile) and k over as many
@@ -846,8 +893,13 @@ void launch_q4k_mode(const WeightDev &w, const float *x, float *y, int flags, co
 // 16 waves 5.5, in 8 6.0; with the norm, 8192 x 2048 4.6 (two tiles 4.6), 16384
 // x 2048 9.1 / 6.2 (one tile 6.4), 40000 x 2048 26 / 11.3, 120818 x 2048 74 /
 // 26.5 (one tile 31.4, four 28.1).
-hipError_t launch_q4k(const WeightDev &w, const float *x, float *y, int flags, const float *nw, float eps,
-                      hipStream_t s) {
+// Q6_K by the same rule, the VALU form / here: 3072 x 2048 + norm 4.0 / 3.5, 2048 x
+// 2048 3.25 / 2.9, 12288 x 2048 + norm + SwiGLU 8.5 / 6.8, 2048 x 6144 5.9 / 4.8,
+// 2048 x 8192 7.1 / 5.5, with the norm 16384 x 2048 10.2 / 7.4, 40000 x 2048
+// 17.8 / 13.6, 120818 x 2048 42.5 / 36.4 (5.6 TB/s).
+template <bool Q6>
+hipError_t launch_kq(const WeightDev &w, const float *x, float *y, int flags, const float *nw, float eps,
+                     hipStream_t s) {
     if (w.cols % 2048 != 0 || w.cols > 8192) return hipErrorInvalidValue;
     const bool glu = flags & kGemvOutSwiGLU;
     const int tiles = glu ? 2 * ((w.rows / 2 + 15) / 16) : (w.rows + 15) / 16;
@@ -855,8 +907,8 @@ hipError_t launch_q4k(const WeightDev &w, const float *x, float *y, int flags, c
     KernelSpan span(gemv_span_name(w.type), s, true);
     auto go = [&](auto waves, auto sbs, int rt) {
         constexpr int NW = decltype(waves)::value, NSB = decltype(sbs)::value;
-        if (rt == 2) launch_q4k_mode<2, NW, NSB>(w, x, y, flags, nw, eps, (tiles + 1) / 2, span, s);
-        else launch_q4k_mode<1, NW, NSB>(w, x, y, flags, nw, eps, tiles, span, s);
+        if (rt == 2) launch_kq_mode<Q6, 2, NW, NSB>(w, x, y, flags, nw, eps, (tiles + 1) / 2, span, s);
+        else launch_kq_mode<Q6, 1, NW, NSB>(w, x, y, flags, nw, eps, tiles, span, s);
     };
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
@@ -917,18 +969,18 @@ hipError_t launch_gemv(const WeightDev &w, const float *x, float *y, int flags, 
     case kW_F32: return launch_t<UnitF32, false>(w, x, y, flags, nw, eps, s);
     case kW_F16: return launch_t<UnitF16, false>(w, x, y, flags, nw, eps, s);
     case kW_Q8_0: return launch_t<UnitQ8_0, false>(w, x, y, flags, nw, eps, s);
-    case kW_Q4_K: return launch_q4k(w, x, y, flags, nw, eps, s);
-    case kW_Q6_K: return launch_t<UnitQ6_K, false>(w, x, y, flags, nw, eps, s);
+    case kW_Q4_K: return launch_kq<false>(w, x, y, flags, nw, eps, s);
+    case kW_Q6_K: return launch_kq<true>(w, x, y, flags, nw, eps, s);
     case kW_Q2_0C: return launch_t<UnitQ2_0C, false>(w, x, y, flags, nw, eps, s);
     case kW_STQ1_0: return launch_t<UnitSTQ1_0, true>(w, x, y, flags, nw, eps, s);
     default: return hipErrorInvalidValue;
     }
 }
 
-hipError_t launch_q4k_tiles(const void *blocks, int rows, int cols, void *tiles, hipStream_t s) {
+hipError_t launch_kq_tiles(int type, const void *blocks, int rows, int cols, void *tiles, hipStream_t s) {
     const int nsb = cols / 256, n = (rows + 15) / 16 * nsb;
-    hipLaunchKernelGGL(q4k_tiles_kernel, dim3((n + 3) / 4), dim3(256), 0, s, (const uint8_t *)blocks, rows, nsb, n,
-                       (uint8_t *)tiles);
+    hipLaunchKernelGGL(type == kW_Q6_K ? q6k_tiles_kernel : q4k_tiles_kernel, dim3((n + 3) / 4), dim3(256), 0, s,
+                       (const uint8_t *)blocks, rows, nsb, n, (uint8_t *)tiles);
     return hipGetLastError();
 }
 

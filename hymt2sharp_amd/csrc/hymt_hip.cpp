@@ -1012,12 +1012,12 @@ struct hymt_weight {
     uint16_t *dense = nullptr;  // bf16 [rows][cols] copy for the prefill GEMMs (hymt_weight_dense)
 };
 
-// A Q4_K matrix into its tiles, through a device buffer of at most 32 MiB that
+// A Q4_K or Q6_K matrix into its tiles, through a device buffer of at most 32 MiB that
 // the call owns (a few rows of tiles at a time), on the null stream as the
 // other types' copy.  Rearranged on the host, the 61-row layer's weights
 // (36 MiB) took 7 ms longer to upload.
-static hipError_t upload_q4k(int rows, int cols, const uint8_t *data, uint8_t *mem) {
-    const size_t rb = (size_t)cols / 256 * 144;
+static hipError_t upload_kq(int type, int rows, int cols, const uint8_t *data, uint8_t *mem) {
+    const size_t rb = (size_t)hymt::gguf_row_bytes(type, cols);
     const int step = (int)std::min<size_t>((32u << 20) / rb / 16 * 16, ((size_t)rows + 15) / 16 * 16);
     uint8_t *tmp = nullptr;
     hipError_t e = hipMalloc((void **)&tmp, rb * (size_t)std::min(step, rows));
@@ -1025,7 +1025,7 @@ static hipError_t upload_q4k(int rows, int cols, const uint8_t *data, uint8_t *m
     for (int r = 0; r < rows && e == hipSuccess; r += std::min(step, rows - r)) {
         const int n = std::min(step, rows - r);
         e = hipMemcpy(tmp, data + rb * (size_t)r, rb * (size_t)n, hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hymt::launch_q4k_tiles(tmp, n, cols, mem + hymt::q4k_tile_bytes(r, cols), nullptr);
+        if (e == hipSuccess) e = hymt::launch_kq_tiles(type, tmp, n, cols, mem + hymt::kq_tile_bytes(type, r, cols), nullptr);
         if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     }
     const hipError_t f = hipFree(tmp);
@@ -1046,11 +1046,11 @@ int hymt_weight_upload(hymt_ctx *c, int type, int rows, int cols, const void *da
     if (bytes != (size_t)rows * (size_t)rb)
         return fail(HYMT_E_ARG, "weight data is " + std::to_string(bytes) + " bytes, expected " +
                                     std::to_string((size_t)rows * (size_t)rb));
-    const bool tiles = type == hymt::kW_Q4_K;  // rearranged on the device; the others on the host
+    const bool tiles = type == hymt::kW_Q4_K || type == hymt::kW_Q6_K;  // rearranged on the device; the others on the host
     hymt::PackedWeight pk;
     if (!tiles && !hymt::pack_weight(type, rows, cols, (const uint8_t *)data, pk))
         return fail(HYMT_E_UNSUPPORTED, "weight type " + std::to_string(type) + " is not supported");
-    const size_t size = tiles ? hymt::q4k_tile_bytes(rows, cols) : pk.buf.size();
+    const size_t size = tiles ? hymt::kq_tile_bytes(type, rows, cols) : pk.buf.size();
     hymt_weight *w = new (std::nothrow) hymt_weight();
     if (!w) return fail(HYMT_E_OOM, "host allocation failed");
     (void)hipSetDevice(c->device);
@@ -1060,7 +1060,7 @@ int hymt_weight_upload(hymt_ctx *c, int type, int rows, int cols, const void *da
         return fail(HYMT_E_OOM, std::string("hipMalloc: ") + hipGetErrorString(e));
     }
     if (tiles)
-        e = upload_q4k(rows, cols, (const uint8_t *)data, (uint8_t *)w->mem);
+        e = upload_kq(type, rows, cols, (const uint8_t *)data, (uint8_t *)w->mem);
     else
         e = hipMemcpy(w->mem, pk.buf.data(), size, hipMemcpyHostToDevice);
     if (e != hipSuccess) {

@@ -79,17 +79,6 @@ bool pack_weight(int type, int rows, int cols, const uint8_t *src, PackedWeight 
         }
         return true;
     }
-    case kW_Q6_K: {  // 210-byte blocks: ql 128, qh 64, scales 16, fp16 d
-        alloc(R * (C / 256) * 208, 0, R * (C / 256) * 4);
-        B = out.buf.data();
-        float *d = (float *)(B + out.off_d);
-        for (size_t b = 0; b < R * (C / 256); b++) {
-            const uint8_t *s = src + 210 * b;
-            std::memcpy(B + 208 * b, s, 208);
-            d[b] = half_to_float(rd16(s + 208));
-        }
-        return true;
-    }
     case kW_Q2_0C: {  // 130-byte blocks: fp16 d, 128 code bytes
         alloc(R * (C / 4), 0, R * (C / 512) * 4);
         B = out.buf.data();

@@ -13,8 +13,12 @@
 //              1024 + 16 lane; at kQ4Scales + 16 c + 4 g the scales of
 //              sub-blocks 2 g and 2 g + 1, then their mins, a byte each; at
 //              kQ4D + 4 c the row's fp16 d and dmin
-//   Q6_K       q: 208-byte super-blocks ql[128] qh[64] scales[16]; d: fp32
-//              [rows][cols/256]
+//   Q6_K       q: tiles alike, kQ6Tile bytes: lane (g, c) holds sub-blocks 4 g + m
+//              (m < 4) of row c, 16 codes each; the low nibbles of m = 0 and 1
+//              (high half of the byte) at 16 lane, of m = 2 and 3 at 1024 +
+//              16 lane, the two high bits at kQ6Hi + 16 lane, bits 6 - 2 m and up,
+//              the upper one flipped; at kQ6Scales + 16 c the 16 scales, at
+//              kQ6D + 2 c the row's fp16 d
 //   Q2_0C      q: the code bytes [rows][cols/4]; d: fp32 [rows][cols/512]
 //   STQ1_0     q: the slot bytes [rows][cols/8]; q2: the sign bytes
 //              [rows][cols/32]; d: fp32 [rows][cols/256]
@@ -32,8 +36,9 @@ namespace hymt {
 // GgmlTensorType codes (GgmlTensorType.cs)
 constexpr int kW_F32 = 0, kW_F16 = 1, kW_Q8_0 = 8, kW_Q4_K = 12, kW_Q6_K = 14, kW_Q2_0C = 40, kW_STQ1_0 = 43;
 
-// the tile of a Q4_K matrix
+// the tiles of a Q4_K and of a Q6_K matrix
 constexpr int kQ4Scales = 2048, kQ4D = kQ4Scales + 256, kQ4Tile = kQ4D + 64;
+constexpr int kQ6Hi = 2048, kQ6Scales = kQ6Hi + 1024, kQ6D = kQ6Scales + 256, kQ6Tile = kQ6D + 32;
 
 struct WeightDev {
     int type, rows, cols;
@@ -51,14 +56,15 @@ struct PackedWeight {
     std::vector<uint8_t> buf;
     size_t off_q = 0, off_q2 = SIZE_MAX, off_d = SIZE_MAX;
 };
-// All types but Q4_K, whose blocks launch_q4k_tiles rearranges on the device.
+// All types but Q4_K and Q6_K, whose blocks launch_kq_tiles rearranges on the
+// device.
 bool pack_weight(int type, int rows, int cols, const uint8_t *src, PackedWeight &out);
-// Bytes of a Q4_K matrix's tiles, and the tiles from its GGUF blocks (both on
-// the device).
-inline size_t q4k_tile_bytes(int rows, int cols) {
-    return (size_t)((rows + 15) / 16) * (cols / 256) * kQ4Tile;
+// Bytes of a Q4_K or Q6_K matrix's tiles, and the tiles from its GGUF blocks
+// (both on the device).
+inline size_t kq_tile_bytes(int type, int rows, int cols) {
+    return (size_t)((rows + 15) / 16) * (cols / 256) * (type == kW_Q6_K ? kQ6Tile : kQ4Tile);
 }
-hipError_t launch_q4k_tiles(const void *blocks, int rows, int cols, void *tiles, hipStream_t s);
+hipError_t launch_kq_tiles(int type, const void *blocks, int rows, int cols, void *tiles, hipStream_t s);
 
 // gemv flags (as HYMT_GEMV_* in include/hymt_hip.h)
 constexpr int kGemvAccumulate = 1, kGemvInRmsNorm = 2, kGemvInSwiGLU = 4, kGemvOutSwiGLU = 8;

@@ -1,5 +1,5 @@
 """The Q4_K GEMV on the matrix cores (hymt2sharp_amd/csrc/gemv.hip,
-gemv_q4k_kernel): every form of its dispatch (waves over 2048 to 8192 columns,
+gemv_kq_kernel): every form of its dispatch (waves over 2048 to 8192 columns,
 one or two 16-row tiles a workgroup), row counts that do not fill a tile,
 the input and output modes, and inputs of extreme range, against the fp64
 product of the dequantized weights.
