@@ -8,7 +8,7 @@
 // decode GEMV moves 1-15 MB, so the kernel is as much about memory latency as
 // bandwidth: a lane issues the loads of all its units before it touches x.
 //
-// Work split of every type but Q4_K and Q6_K, which run on the matrix cores
+// Work split of every type but Q4_K, Q6_K and Q8_0, which run on the matrix cores
 // (gemv_kq_kernel): 256 threads (4 waves).  A row takes a group of LPR lanes (8..64,
 // a power of two); lane j of the group handles units j + LPR k (k < K =
 // UPR / LPR, UPR = cols / 32 units per row), so neighbouring lanes read
@@ -135,36 +135,25 @@ struct UnitF16 {
     }
 };
 
-// Q8_0 (Q8_0.cs:16-35): q int8 [rows][cols], d fp32 [rows][cols/32]
+// Q8_0 (Q8_0.cs:16-35) in the tiles of weights.hpp, dequantized.  Unit u is
+// block u%8 of 256 columns: g = (u%8)/2, its 16-value halves m = 2 (u%2) and the
+// next.
 struct UnitQ8_0 {
-    static constexpr int kMax = 8;  // units in flight per lane
     uint4 v[2];
     float d;
     __device__ void load(const WeightDev &w, int r, int u) {
-        const uint4 *p = (const uint4 *)((const int8_t *)w.q + (size_t)r * w.cols + 32 * u);
-        v[0] = p[0];
-        v[1] = p[1];
-        d = w.d[(size_t)r * (w.cols / 32) + u];
-    }
-    __device__ float dot(const WeightDev &, int, int u, const float *x, const float *) const {
-        const float4 *xv = (const float4 *)(x + xpad(32 * u));
-        float a = 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const uint32_t wd = i < 4 ? (&v[0].x)[i] : (&v[1].x)[i - 4];
-            const float q[4] = {(float)(int8_t)(wd & 0xFF), (float)(int8_t)((wd >> 8) & 0xFF),
-                                (float)(int8_t)((wd >> 16) & 0xFF), (float)(int8_t)(wd >> 24)};
-            a = dot4(q, xv[i], a);
-        }
-        return d * a;
+        const int sub = u & 7, lane = (sub >> 1) * 16 + (r & 15);
+        const uint8_t *b = (const uint8_t *)w.q + ((size_t)(r >> 4) * (w.cols / 256) + (u >> 3)) * kQ8Tile;
+        v[0] = *(const uint4 *)(b + 2048 * (sub & 1) + 16 * lane);
+        v[1] = *(const uint4 *)(b + 2048 * (sub & 1) + 1024 + 16 * lane);
+        d = h2f(*(const uint16_t *)(b + kQ8D + 16 * (r & 15) + 2 * sub));
     }
     __device__ void store(int u, float, float *o) const {
+        const uint32_t wd[8] = {v[0].x, v[0].y, v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w};
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const uint32_t wd = i < 4 ? (&v[0].x)[i] : (&v[1].x)[i - 4];
+        for (int i = 0; i < 8; i++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) o[32 * u + 4 * i + e] = d * (float)(int8_t)((wd >> (8 * e)) & 0xFF);
-        }
+            for (int e = 0; e < 4; e++) o[32 * u + 4 * i + e] = d * (float)(int8_t)(wd[i] >> (8 * e));
     }
 };
 
@@ -480,7 +469,7 @@ __global__ __launch_bounds__(256) void embed_kernel(WeightDev w, int row, float 
     }
 }
 
-// ---- Q4_K and Q6_K on the matrix cores -------------------------------------------
+// ---- Q4_K, Q6_K and Q8_0 on the matrix cores --------------------------------------
 // y = W x' for Q4_K, in integers.  The VALU form of the other types spends a
 // convert and an fma per weight, the scales' bit fields, and x and its sums
 // staged by every workgroup behind two barriers: on 120818 x 2048 rows 74 us
@@ -517,6 +506,13 @@ __global__ __launch_bounds__(256) void embed_kernel(WeightDev w, int row, float 
 // 1.3e-7), log-normal 0.7e-7 to 0.9e-7 (1.3e-7), all positive 0.7e-7 (1.1e-7 to
 // 1.7e-7).
 //
+// Q8_0's codes are the B operand's bytes as they are; a lane (p, c) receives the
+// sums over blocks 2 g and 2 g + 1 as with Q4_K, below 2^20 and so exact in
+// fp32, where the blocks' fp16 scales meet them.  rms
+// error: normal x 0.9e-7 to 1.0e-7 (1.3e-7), outliers 0.6e-7 to 0.9e-7 (1.4e-7 to
+// 1.6e-7), log-normal 0.7e-7 to 0.9e-7 (1.2e-7 to 1.4e-7), all positive 0.8e-7 to
+// 1.0e-7 (1.2e-7).
+//
 // Work split: a workgroup of NW waves takes RT tiles of 16 rows; wave v takes
 // super-blocks [v NSB, (v + 1) NSB) of all of them, whose x' it prepares for
 // itself in LDS, so nothing waits for another wave until the partial sums of a
@@ -549,11 +545,12 @@ __device__ __forceinline__ void wave_order() {
     __builtin_amdgcn_wave_barrier();
 }
 
-template <bool Q6, int RT, int NW, int NSB, int MODE>
+template <int T, int RT, int NW, int NSB, int MODE>
 __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const float *__restrict__ xg,
                                                           float *__restrict__ y, int flags,
                                                           const float *__restrict__ nw, float eps) {
-    constexpr int kTile = Q6 ? kQ6Tile : kQ4Tile;
+    constexpr bool Q6 = T == kW_Q6_K, Q8 = T == kW_Q8_0;
+    constexpr int kTile = Q8 ? kQ8Tile : Q6 ? kQ6Tile : kQ4Tile;
     // a wave's super-blocks as digits, [group][digit][64 columns], and zeros
     __shared__ __attribute__((aligned(16))) uint8_t s_x[NW][NSB + 1][1024];
     __shared__ float s_p[NW][RT][16];
@@ -574,7 +571,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
     }
     // tile i's row of this lane; with SwiGLU the tiles alternate between gate
     // rows and the same rows of up
-    uint4 q0[RT][NSB], q1[RT][NSB], qh[RT][NSB], sm[RT][NSB];
+    uint4 q0[RT][NSB], q1[RT][NSB], q2[RT][NSB], q3[RT][NSB], sm[RT][NSB];
     uint32_t dd[RT][NSB];
 #pragma unroll
     for (int i = 0; i < RT; i++) {
@@ -587,8 +584,12 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
         for (int s = 0; s < NSB; s++) {
             q0[i][s] = *(const uint4 *)(b + s * kTile + 16 * li);
             q1[i][s] = *(const uint4 *)(b + s * kTile + 1024 + 16 * li);
-            if constexpr (Q6) {
-                qh[i][s] = *(const uint4 *)(b + s * kTile + kQ6Hi + 16 * li);
+            if constexpr (Q8) {
+                q2[i][s] = *(const uint4 *)(b + s * kTile + 2048 + 16 * li);
+                q3[i][s] = *(const uint4 *)(b + s * kTile + 3072 + 16 * li);
+                sm[i][s] = *(const uint4 *)(b + s * kTile + kQ8D + 16 * r);
+            } else if constexpr (Q6) {
+                q2[i][s] = *(const uint4 *)(b + s * kTile + kQ6Hi + 16 * li);
                 sm[i][s] = *(const uint4 *)(b + s * kTile + kQ6Scales + 16 * r);
                 dd[i][s] = *(const uint16_t *)(b + s * kTile + kQ6D + 2 * r);
             } else {
@@ -615,7 +616,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
 #pragma unroll
             for (int e = 0; e < 4; e++) v[e] = v[e] / (1.f + expf(-v[e])) * g[e];
         }
-        if constexpr (!Q6) {  // sums over the sub-blocks (8 lanes) of this lane group: 2 grp, 2 grp + 1
+        if constexpr (!Q6 && !Q8) {  // sums over the sub-blocks (8 lanes) of this lane group: 2 grp, 2 grp + 1
             float a = (v[0] + v[1]) + (v[2] + v[3]);
             a += dpp<0xB1>(a);
             a += dpp<0x4E>(a);
@@ -637,7 +638,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
         const int e = min(max((int)(mx >> 23), 30), 254);
         const float sc = __uint_as_float((uint32_t)(283 - e) << 23);
         wgt[s] = __uint_as_float((uint32_t)(e - 29 + 8 * grp) << 23);  // of digit `grp`
-        if (Q6 && mx >= 0x7F800000u) wgt[s] = NAN;
+        if ((Q6 || Q8) && mx >= 0x7F800000u) wgt[s] = NAN;
         // four signed digits of each column: with 0x80 added to the lower
         // three bytes they are the bytes less 0x80
         uint32_t t[4];
@@ -664,8 +665,26 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
         for (int i = 0; i < RT; i++) {
             const uint4 a = q0[i][s], b = q1[i][s];
             const uint32_t k[4] = {sm[i][s].x, sm[i][s].y, sm[i][s].z, sm[i][s].w};
+            if constexpr (Q8) {
+                const uint4 e = q2[i][s], f = q3[i][s];
+                const i32x4 l0 = {(int)a.x, (int)a.y, (int)a.z, (int)a.w}, l1 = {(int)b.x, (int)b.y, (int)b.z, (int)b.w};
+                const i32x4 h0 = {(int)e.x, (int)e.y, (int)e.z, (int)e.w}, h1 = {(int)f.x, (int)f.y, (int)f.z, (int)f.w};
+                i32x4 L = {0, 0, 0, 0}, H = {0, 0, 0, 0};
+                L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[0], l0, L, 0, 0, 0);
+                H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[2], h0, H, 0, 0, 0);
+                L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[1], l1, L, 0, 0, 0);
+                H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[3], h1, H, 0, 0, 0);
+                float t = 0.f;
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    t = fmaf(h2f(k[g] & 0xFFFF), (float)L[g], t);
+                    t = fmaf(h2f(k[g] >> 16), (float)H[g], t);
+                }
+                acc[i] = fmaf(t, wgt[s], acc[i]);
+                continue;
+            }
             if constexpr (Q6) {
-                const uint32_t h[4] = {qh[i][s].x, qh[i][s].y, qh[i][s].z, qh[i][s].w};
+                const uint32_t h[4] = {q2[i][s].x, q2[i][s].y, q2[i][s].z, q2[i][s].w};
                 const uint32_t lo[2][4] = {{a.x, a.y, a.z, a.w}, {b.x, b.y, b.z, b.w}};
                 int t = 0;
 #pragma unroll
@@ -810,6 +829,30 @@ __global__ __launch_bounds__(256) void q6k_tiles_kernel(const uint8_t *__restric
     if (g == 0) *(uint16_t *)(t + kQ6D + 2 * c) = (uint16_t)d;
 }
 
+// The same for Q8_0's GGUF blocks (fp16 d, 32 int8: 34 bytes, 2-byte aligned).
+__global__ __launch_bounds__(256) void q80_tiles_kernel(const uint8_t *__restrict__ blocks, int rows, int nsb, int tiles,
+                                                        uint8_t *__restrict__ out) {
+    const int tile = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    if (tile >= tiles) return;
+    const int row = tile / nsb * 16 + c, sb = tile % nsb;
+    uint32_t q[4][4] = {}, d = 0;
+    if (row < rows) {
+        const uint8_t *b = blocks + (((size_t)row * nsb + sb) * 8 + 2 * g) * 34;
+        auto rd = [&](int at) {  // 4 bytes, 2-byte aligned
+            return *(const uint16_t *)(b + at) | (uint32_t)*(const uint16_t *)(b + at + 2) << 16;
+        };
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) q[m][i] = rd(34 * (m >> 1) + 2 + 16 * (m & 1) + 4 * i);
+        d = *(const uint16_t *)b | (uint32_t)*(const uint16_t *)(b + 34) << 16;
+    }
+    uint8_t *t = out + (size_t)tile * kQ8Tile;
+#pragma unroll
+    for (int m = 0; m < 4; m++) *(uint4 *)(t + 1024 * m + 16 * lane) = make_uint4(q[m][0], q[m][1], q[m][2], q[m][3]);
+    *(uint32_t *)(t + kQ8D + 16 * c + 4 * g) = d;
+}
+
 const char *gemv_span_name(int type) {
     switch (type) {
     case kW_F32: return "gemv_f32";
@@ -874,13 +917,13 @@ hipError_t launch_t(const WeightDev &w, const float *x, float *y, int flags, con
     return hipGetLastError();
 }
 
-template <bool Q6, int RT, int NW, int NSB>
+template <int T, int RT, int NW, int NSB>
 void launch_kq_mode(const WeightDev &w, const float *x, float *y, int flags, const float *nw, float eps, int grid,
                     const KernelSpan &span, hipStream_t s) {
     const dim3 g(grid), b(64 * NW);
-    if (flags & kGemvInRmsNorm) launch(span, gemv_kq_kernel<Q6, RT, NW, NSB, 1>, g, b, 0, s, w, x, y, flags, nw, eps);
-    else if (flags & kGemvInSwiGLU) launch(span, gemv_kq_kernel<Q6, RT, NW, NSB, 2>, g, b, 0, s, w, x, y, flags, nw, eps);
-    else launch(span, gemv_kq_kernel<Q6, RT, NW, NSB, 0>, g, b, 0, s, w, x, y, flags, nw, eps);
+    if (flags & kGemvInRmsNorm) launch(span, gemv_kq_kernel<T, RT, NW, NSB, 1>, g, b, 0, s, w, x, y, flags, nw, eps);
+    else if (flags & kGemvInSwiGLU) launch(span, gemv_kq_kernel<T, RT, NW, NSB, 2>, g, b, 0, s, w, x, y, flags, nw, eps);
+    else launch(span, gemv_kq_kernel<T, RT, NW, NSB, 0>, g, b, 0, s, w, x, y, flags, nw, eps);
 }
 
 // One tile per workgroup (with SwiGLU a gate and an up tile) and k over as many
@@ -897,7 +940,10 @@ void launch_kq_mode(const WeightDev &w, const float *x, float *y, int flags, con
 // 2048 3.25 / 2.9, 12288 x 2048 + norm + SwiGLU 8.5 / 6.8, 2048 x 6144 5.9 / 4.8,
 // 2048 x 8192 7.1 / 5.5, with the norm 16384 x 2048 10.2 / 7.4, 40000 x 2048
 // 17.8 / 13.6, 120818 x 2048 42.5 / 36.4 (5.6 TB/s).
-template <bool Q6>
+// Q8_0 likewise (its VALU form had a byte convert and an fma per weight and fp32
+// scales): 4.0 / 3.7, 3.1 / 2.7, 7.3 / 7.4, 5.7 / 4.8, 6.9 / 5.8, 9.4 / 8.4, 18.1 /
+// 17.8, 47.5 / 46.5 (5.65 TB/s).
+template <int T>
 hipError_t launch_kq(const WeightDev &w, const float *x, float *y, int flags, const float *nw, float eps,
                      hipStream_t s) {
     if (w.cols % 2048 != 0 || w.cols > 8192) return hipErrorInvalidValue;
@@ -907,8 +953,8 @@ hipError_t launch_kq(const WeightDev &w, const float *x, float *y, int flags, co
     KernelSpan span(gemv_span_name(w.type), s, true);
     auto go = [&](auto waves, auto sbs, int rt) {
         constexpr int NW = decltype(waves)::value, NSB = decltype(sbs)::value;
-        if (rt == 2) launch_kq_mode<Q6, 2, NW, NSB>(w, x, y, flags, nw, eps, (tiles + 1) / 2, span, s);
-        else launch_kq_mode<Q6, 1, NW, NSB>(w, x, y, flags, nw, eps, tiles, span, s);
+        if (rt == 2) launch_kq_mode<T, 2, NW, NSB>(w, x, y, flags, nw, eps, (tiles + 1) / 2, span, s);
+        else launch_kq_mode<T, 1, NW, NSB>(w, x, y, flags, nw, eps, tiles, span, s);
     };
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
@@ -968,9 +1014,9 @@ hipError_t launch_gemv(const WeightDev &w, const float *x, float *y, int flags, 
     switch (w.type) {
     case kW_F32: return launch_t<UnitF32, false>(w, x, y, flags, nw, eps, s);
     case kW_F16: return launch_t<UnitF16, false>(w, x, y, flags, nw, eps, s);
-    case kW_Q8_0: return launch_t<UnitQ8_0, false>(w, x, y, flags, nw, eps, s);
-    case kW_Q4_K: return launch_kq<false>(w, x, y, flags, nw, eps, s);
-    case kW_Q6_K: return launch_kq<true>(w, x, y, flags, nw, eps, s);
+    case kW_Q8_0: return launch_kq<kW_Q8_0>(w, x, y, flags, nw, eps, s);
+    case kW_Q4_K: return launch_kq<kW_Q4_K>(w, x, y, flags, nw, eps, s);
+    case kW_Q6_K: return launch_kq<kW_Q6_K>(w, x, y, flags, nw, eps, s);
     case kW_Q2_0C: return launch_t<UnitQ2_0C, false>(w, x, y, flags, nw, eps, s);
     case kW_STQ1_0: return launch_t<UnitSTQ1_0, true>(w, x, y, flags, nw, eps, s);
     default: return hipErrorInvalidValue;
@@ -979,8 +1025,8 @@ hipError_t launch_gemv(const WeightDev &w, const float *x, float *y, int flags, 
 
 hipError_t launch_kq_tiles(int type, const void *blocks, int rows, int cols, void *tiles, hipStream_t s) {
     const int nsb = cols / 256, n = (rows + 15) / 16 * nsb;
-    hipLaunchKernelGGL(type == kW_Q6_K ? q6k_tiles_kernel : q4k_tiles_kernel, dim3((n + 3) / 4), dim3(256), 0, s,
-                       (const uint8_t *)blocks, rows, nsb, n, (uint8_t *)tiles);
+    hipLaunchKernelGGL(type == kW_Q8_0 ? q80_tiles_kernel : type == kW_Q6_K ? q6k_tiles_kernel : q4k_tiles_kernel,
+                       dim3((n + 3) / 4), dim3(256), 0, s, (const uint8_t *)blocks, rows, nsb, n, (uint8_t *)tiles);
     return hipGetLastError();
 }
 

@@ -1012,7 +1012,7 @@ struct hymt_weight {
     uint16_t *dense = nullptr;  // bf16 [rows][cols] copy for the prefill GEMMs (hymt_weight_dense)
 };
 
-// A Q4_K or Q6_K matrix into its tiles, through a device buffer of at most 32 MiB that
+// A Q4_K, Q6_K or Q8_0 matrix into its tiles, through a device buffer of at most 32 MiB that
 // the call owns (a few rows of tiles at a time), on the null stream as the
 // other types' copy.  Rearranged on the host, the 61-row layer's weights
 // (36 MiB) took 7 ms longer to upload.
@@ -1046,7 +1046,8 @@ int hymt_weight_upload(hymt_ctx *c, int type, int rows, int cols, const void *da
     if (bytes != (size_t)rows * (size_t)rb)
         return fail(HYMT_E_ARG, "weight data is " + std::to_string(bytes) + " bytes, expected " +
                                     std::to_string((size_t)rows * (size_t)rb));
-    const bool tiles = type == hymt::kW_Q4_K || type == hymt::kW_Q6_K;  // rearranged on the device; the others on the host
+    // rearranged on the device; the others on the host
+    const bool tiles = type == hymt::kW_Q4_K || type == hymt::kW_Q6_K || type == hymt::kW_Q8_0;
     hymt::PackedWeight pk;
     if (!tiles && !hymt::pack_weight(type, rows, cols, (const uint8_t *)data, pk))
         return fail(HYMT_E_UNSUPPORTED, "weight type " + std::to_string(type) + " is not supported");

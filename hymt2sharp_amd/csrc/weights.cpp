@@ -68,17 +68,6 @@ bool pack_weight(int type, int rows, int cols, const uint8_t *src, PackedWeight 
         alloc(R * rb, 0, 0);
         std::memcpy(out.buf.data(), src, R * rb);
         return true;
-    case kW_Q8_0: {  // 34-byte blocks: fp16 d, 32 int8
-        alloc(R * C, 0, R * (C / 32) * 4);
-        B = out.buf.data();
-        float *d = (float *)(B + out.off_d);
-        for (size_t b = 0; b < R * (C / 32); b++) {
-            const uint8_t *s = src + 34 * b;
-            d[b] = half_to_float(rd16(s));
-            std::memcpy(B + 32 * b, s + 2, 32);
-        }
-        return true;
-    }
     case kW_Q2_0C: {  // 130-byte blocks: fp16 d, 128 code bytes
         alloc(R * (C / 4), 0, R * (C / 512) * 4);
         B = out.buf.data();

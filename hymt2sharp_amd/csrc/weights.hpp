@@ -5,7 +5,6 @@
 // BlockLayout.cs:9-106).  hymt_weight_upload repacks it so that every 32-value
 // unit of a row is read with aligned vector loads:
 //   F32, F16   as stored, [rows][cols]
-//   Q8_0       q: int8 [rows][cols]; d: fp32 [rows][cols/32]
 //   Q4_K       q: tiles of 16 rows (the last one padded with zeros) x one
 //              super-block of 256 columns, kQ4Tile bytes, [row / 16][cols / 256]:
 //              the code bytes as lane (g, c) = 16 g + c of a wave reads them,
@@ -19,6 +18,9 @@
 //              16 lane, the two high bits at kQ6Hi + 16 lane, bits 6 - 2 m and up,
 //              the upper one flipped; at kQ6Scales + 16 c the 16 scales, at
 //              kQ6D + 2 c the row's fp16 d
+//   Q8_0       q: tiles alike, kQ8Tile bytes: lane (g, c) holds columns 64 g + 16 m
+//              + [0, 16) of row c at 1024 m + 16 lane (m < 4); at kQ8D + 16 c the
+//              row's 8 fp16 scales
 //   Q2_0C      q: the code bytes [rows][cols/4]; d: fp32 [rows][cols/512]
 //   STQ1_0     q: the slot bytes [rows][cols/8]; q2: the sign bytes
 //              [rows][cols/32]; d: fp32 [rows][cols/256]
@@ -36,9 +38,10 @@ namespace hymt {
 // GgmlTensorType codes (GgmlTensorType.cs)
 constexpr int kW_F32 = 0, kW_F16 = 1, kW_Q8_0 = 8, kW_Q4_K = 12, kW_Q6_K = 14, kW_Q2_0C = 40, kW_STQ1_0 = 43;
 
-// the tiles of a Q4_K and of a Q6_K matrix
+// the tiles of a Q4_K, a Q6_K and a Q8_0 matrix
 constexpr int kQ4Scales = 2048, kQ4D = kQ4Scales + 256, kQ4Tile = kQ4D + 64;
 constexpr int kQ6Hi = 2048, kQ6Scales = kQ6Hi + 1024, kQ6D = kQ6Scales + 256, kQ6Tile = kQ6D + 32;
+constexpr int kQ8D = 4096, kQ8Tile = kQ8D + 256;
 
 struct WeightDev {
     int type, rows, cols;
@@ -56,13 +59,13 @@ struct PackedWeight {
     std::vector<uint8_t> buf;
     size_t off_q = 0, off_q2 = SIZE_MAX, off_d = SIZE_MAX;
 };
-// All types but Q4_K and Q6_K, whose blocks launch_kq_tiles rearranges on the
+// All types but Q4_K, Q6_K and Q8_0, whose blocks launch_kq_tiles rearranges on the
 // device.
 bool pack_weight(int type, int rows, int cols, const uint8_t *src, PackedWeight &out);
-// Bytes of a Q4_K or Q6_K matrix's tiles, and the tiles from its GGUF blocks
+// Bytes of such a matrix's tiles, and the tiles from its GGUF blocks
 // (both on the device).
 inline size_t kq_tile_bytes(int type, int rows, int cols) {
-    return (size_t)((rows + 15) / 16) * (cols / 256) * (type == kW_Q6_K ? kQ6Tile : kQ4Tile);
+    return (size_t)((rows + 15) / 16) * (cols / 256) * (type == kW_Q8_0 ? kQ8Tile : type == kW_Q6_K ? kQ6Tile : kQ4Tile);
 }
 hipError_t launch_kq_tiles(int type, const void *blocks, int rows, int cols, void *tiles, hipStream_t s);
 
