@@ -570,13 +570,14 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
         if constexpr (MODE == 2) gv[s] = ((const float4 *)(xg + w.cols))[(sb0 + s) * 64 + lane];
     }
     // tile i's row of this lane; with SwiGLU the tiles alternate between gate
-    // rows and the same rows of up
+    // rows and the same rows of up, or (RT = 1) a tile is 8 of each
     uint4 q0[RT][NSB], q1[RT][NSB], q2[RT][NSB], q3[RT][NSB], sm[RT][NSB];
     uint32_t dd[RT][NSB];
 #pragma unroll
     for (int i = 0; i < RT; i++) {
-        const int row = min(out_swiglu ? (i & 1) * F + 16 * ((int)(blockIdx.x * RT + i) >> 1) + c
-                                       : 16 * (int)(blockIdx.x * RT + i) + c,
+        const int row = min(out_swiglu && RT == 1 ? (c >> 3) * F + 8 * (int)blockIdx.x + (c & 7)
+                            : out_swiglu          ? (i & 1) * F + 16 * ((int)(blockIdx.x * RT + i) >> 1) + c
+                                                  : 16 * (int)(blockIdx.x * RT + i) + c,
                             w.rows - 1);
         const int r = row & 15, li = grp * 16 + r;
         const uint8_t *b = (const uint8_t *)w.q + ((size_t)(row >> 4) * nsb + sb0) * kTile;
@@ -750,9 +751,9 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
     };
     const int i = tid >> 4, r = tid & 15;
     if (out_swiglu) {
-        const int o = 16 * ((int)(blockIdx.x * RT >> 1) + i) + r;
+        const int o = RT == 1 ? 8 * (int)blockIdx.x + r : 16 * ((int)(blockIdx.x * RT >> 1) + i) + r;
         if (o >= F) return;
-        const float gt = sum(2 * i, r), up = sum(2 * i + 1, r);
+        const float gt = RT == 1 ? sum(0, r) : sum(2 * i, r), up = RT == 1 ? sum(0, 8 + r) : sum(2 * i + 1, r);
         y[o] = gt / (1.f + expf(-gt)) * up;  // Ops.SiLUMul (Ops.cs:1016-1052)
         return;
     }
@@ -941,20 +942,24 @@ void launch_kq_mode(const WeightDev &w, const float *x, float *y, int flags, con
 // 2048 x 8192 7.1 / 5.5, with the norm 16384 x 2048 10.2 / 7.4, 40000 x 2048
 // 17.8 / 13.6, 120818 x 2048 42.5 / 36.4 (5.6 TB/s).
 // Q8_0 likewise (its VALU form had a byte convert and an fma per weight and fp32
-// scales): 4.0 / 3.7, 3.1 / 2.7, 7.3 / 7.4, 5.7 / 4.8, 6.9 / 5.8, 9.4 / 8.4, 18.1 /
-// 17.8, 47.5 / 46.5 (5.65 TB/s).
+// scales): 4.0 / 3.7, 3.1 / 2.7, 7.3 / 7.1, 5.7 / 4.8, 6.9 / 5.8, 9.4 / 8.4, 18.1 /
+// 17.8, 47.5 / 46.5 (5.65 TB/s).  With SwiGLU Q8_0 takes tiles of 8 gate and 8 up
+// rows, twice the workgroups (768 rather than 384 for 12288 rows, three per CU):
+// half a tile's codes are whole 128-byte lines, as its 4352 bytes are 34 lines.
+// One token through eight layers 164.0 -> 160.0 us; the other types' tiles start
+// within a line, and halves cost them (Q6_K 161.6 -> 169.5, Q4_K 149.1 -> 151.3).
 template <int T>
 hipError_t launch_kq(const WeightDev &w, const float *x, float *y, int flags, const float *nw, float eps,
                      hipStream_t s) {
     if (w.cols % 2048 != 0 || w.cols > 8192) return hipErrorInvalidValue;
     const bool glu = flags & kGemvOutSwiGLU;
     const int tiles = glu ? 2 * ((w.rows / 2 + 15) / 16) : (w.rows + 15) / 16;
-    const bool few = (glu ? tiles / 2 : tiles) <= 512;
+    const bool few = (glu ? tiles / 2 : tiles) <= 512, half = T == kW_Q8_0 && glu && few;
     KernelSpan span(gemv_span_name(w.type), s, true);
     auto go = [&](auto waves, auto sbs, int rt) {
         constexpr int NW = decltype(waves)::value, NSB = decltype(sbs)::value;
         if (rt == 2) launch_kq_mode<T, 2, NW, NSB>(w, x, y, flags, nw, eps, (tiles + 1) / 2, span, s);
-        else launch_kq_mode<T, 1, NW, NSB>(w, x, y, flags, nw, eps, tiles, span, s);
+        else launch_kq_mode<T, 1, NW, NSB>(w, x, y, flags, nw, eps, half ? (w.rows / 2 + 7) / 8 : tiles, span, s);
     };
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
@@ -963,7 +968,7 @@ hipError_t launch_kq(const WeightDev &w, const float *x, float *y, int flags, co
     using I8 = std::integral_constant<int, 8>;
     using I12 = std::integral_constant<int, 12>;
     using I16 = std::integral_constant<int, 16>;
-    const int rt = glu || !few ? 2 : 1;
+    const int rt = half || (!glu && few) ? 1 : 2;
     switch (w.cols / 2048) {
     case 1: go(I8{}, I1{}, rt); break;
     case 2: few ? go(I16{}, I1{}, rt) : go(I8{}, I2{}, rt); break;
