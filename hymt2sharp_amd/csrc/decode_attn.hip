@@ -295,7 +295,7 @@ template <typename S, int VS> struct PageOps {
 //   row to the cache at the end.  So no workgroup is spent on a page that
 //   holds only the new token (L = 4097 runs exactly 256 workgroups).
 // PAGES_ARG: page ids come from the kernel arguments, else from the device
-// page table; both are scalar loads issued first.
+// page table; both are scalar loads, those of the first run issued first.
 // NG: groups of 4 waves in the workgroup.  NG = 1 is the split form above.
 //   NG > 1 is the one-launch form for short caches (nsplit = 1): group g takes
 //   pages g PPW .. of every run of NG PPW pages, and the groups' partials meet
@@ -372,8 +372,14 @@ __global__ __launch_bounds__(256 * NG) void decode_attn_mfma_kernel(DecodeArgs a
     const int plast = max(page_end - 1, page0);
     const bool last = split == nsplit - 1;
     const size_t page_elems = (size_t)P * D;
-    // a page of the device table (wave-uniform), clamped to the split
-    auto tab_page = [&](int p) { return __builtin_amdgcn_readfirstlane(tab[min(p, plast)]); };
+    // page p of the device table, or of the argument list (wave-uniform),
+    // clamped to the split.  A call takes all its pages from one of the two:
+    // the device table may lag behind the list (a page mapped in a recording
+    // that has not run), and a replay repeats the recorded list.
+    auto tab_page = [&](int p) {
+        return PAGES_ARG ? a.pages[min(p, min(plast, kArgPages - 1))]
+                         : __builtin_amdgcn_readfirstlane(tab[min(p, plast)]);
+    };
     auto page_base = [&](int phys) { return ((size_t)phys * Hkv + kvh) * page_elems; };
 
     // ---- 1. every vector load, straight-line: the q row of head kvh*4 +

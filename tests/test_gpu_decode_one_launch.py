@@ -11,6 +11,7 @@ from hymt2sharp_amd._native import BF16, F16, F32
 from tests.attn_cases import BASE, D, EPS, HKV, HQ, cache_rows, max_rel, new_token
 from tests.test_gpu_random_sweep import decode_case
 from tests.test_gpu_decode import ulp_close
+from tests.test_gpu_graph import dev_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +51,36 @@ def test_pages_out_of_order(hip_available, dtype):
             be.Dispose()
     assert outs[0][0] != outs[1][0]
     assert np.array_equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("dtype,pos", [(F32, 180), (F16, 180), (BF16, 350), (F16, 500)])
+def test_replay_keeps_its_pages(hip_available, dtype, pos):
+    """A recorded call takes the page of every run from its arguments: the
+    table may have moved on by the time it is replayed."""
+    kb, vb = cache_rows(17, pos, salt=5)
+    q, k, v, qnw, knw = new_token(17, 5, "gamma")
+    be = HipBackend(0).configure(HQ, HKV, D, D, BASE, EPS).create_cache(1, 640, dtype)
+    try:
+        be.UploadKv(0, 0, pos, kb, vb)
+        ptrs = dev_inputs(be, [q, k, v, qnw, knw])
+        dout = be.alloc(q.nbytes)
+
+        def out():
+            be.sync()
+            return be.download(np.empty(HQ * D, np.float32), dout)
+
+        be.decode_dev(0, pos, *ptrs, dout)
+        eager = out()
+        be.graph_begin()
+        be.decode_dev(0, pos, *ptrs, dout)
+        g = be.graph_end()
+        pages = [be.page_of(b) for b in range(pos // 64 + 1)]
+        be.SetCacheLen(64)                # blocks 1 and up give their pages back
+        be.MapRange(64, pos + 1 - 64)     # and get them again, the last given back first
+        assert [be.page_of(b) for b in range(pos // 64 + 1)] == pages[:1] + pages[:0:-1]
+        be.upload(dout, np.zeros_like(q))
+        be.graph_launch(g)
+        assert np.array_equal(out(), eager)
+        be.graph_destroy(g)
+    finally:
+        be.Dispose()
