@@ -151,6 +151,7 @@ struct hymt_graph {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     uint64_t gen = 0;  // the context's buffer generation at recording
+    std::vector<int> tab;  // page-table entries that a replay writes
 };
 
 namespace {
@@ -164,10 +165,14 @@ int map_hip(const HipError &e) {
 // Mirror changed page-table entries to the device table.
 void flush_table(hymt_ctx *c) {
     if (!c->pages.has_dirty()) return;
-    std::vector<int> idx = c->pages.take_dirty();
+    std::vector<int> idx = c->pages.take_dirty(c->capturing);
     std::vector<int> val(idx.size());
     for (size_t i = 0; i < idx.size(); i++) val[i] = c->pages.phys(idx[i]);
-    HIP_TRY(launch_tab_update((int32_t *)c->tab.p, idx.data(), val.data(), (int)idx.size(), c->stream));
+    const hipError_t e = launch_tab_update((int32_t *)c->tab.p, idx.data(), val.data(), (int)idx.size(), c->stream);
+    if (e != hipSuccess) {
+        c->pages.mark_dirty(idx);
+        HIP_TRY(e);
+    }
 }
 
 // Map [pos, pos+len) for writing: pages for unmapped blocks, fresh pages for
@@ -526,6 +531,7 @@ int hymt_kv_read(hymt_ctx *c, int layer, int pos, int len, float *k_out, float *
     if (int r = refuse_in_capture(c, "hymt_kv_read")) return r;
     try {
         HIP_TRY(hipSetDevice(c->device));
+        flush_table(c);
         const size_t n = (size_t)len * c->kv_heads * c->head_dim;
         c->out_o.reserve(2 * n * 4);
         float *dk = (float *)c->out_o.p, *dv = dk + n;
@@ -947,6 +953,7 @@ int hymt_graph_end(hymt_ctx *c, hymt_graph **out) {
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     c->capturing = false;
+    std::vector<int> tab = c->pages.end_recording();
     if (c->capture_failed || e != hipSuccess || !g) {
         if (g) (void)hipGraphDestroy(g);
         if (e != hipSuccess)
@@ -960,6 +967,7 @@ int hymt_graph_end(hymt_ctx *c, hymt_graph **out) {
     }
     hg->graph = g;
     hg->gen = c->gen;
+    hg->tab = std::move(tab);
     e = hipGraphInstantiate(&hg->exec, g, nullptr, nullptr, 0);
     if (e != hipSuccess) {
         (void)hipGraphDestroy(g);
@@ -981,6 +989,7 @@ int hymt_graph_launch(hymt_ctx *c, hymt_graph *g) {
     TimedCall timed(call_timer(c), "graph_launch", 0);
     KernelSpan span("graph", c->stream);
     hipError_t e = hipGraphLaunch(g->exec, c->stream);
+    c->pages.mark_dirty(g->tab);  // the table has moved on since the recording, perhaps
     if (e != hipSuccess) return fail(HYMT_E_DEVICE, std::string("hipGraphLaunch: ") + hipGetErrorString(e));
     return HYMT_OK;
 }

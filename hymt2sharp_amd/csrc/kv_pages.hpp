@@ -58,7 +58,9 @@ class KvPages {
         : max_pages_((max_tokens + kPageTokens - 1) / kPageTokens),
           tab_(max_pages_, -1),
           refs_(max_pages_, 0),
-          dirty_flag_(max_pages_, 0) {}
+          dirty_flag_(max_pages_, 0) {
+        dirty_.reserve(max_pages_);  // marking an entry allocates nothing
+    }
 
     static uint64_t chain_hash(uint64_t prev, const int32_t *tokens, int n) {
         uint64_t h = prev;
@@ -190,14 +192,32 @@ class KvPages {
         return hit * kPageTokens;
     }
 
-    // Entries changed since the last take_dirty(); clears the list.
-    std::vector<int> take_dirty() {
-        std::vector<int> d;
-        d.swap(dirty_);
+    // Entries changed since the last take_dirty(); clears the list.  When
+    // their update goes into a recording (`recorded`) it reaches the device
+    // table only once, and each time, the recording runs: the owner then says
+    // so with end_recording().
+    std::vector<int> take_dirty(bool recorded = false) {
+        std::vector<int> d(dirty_);
+        if (recorded) recorded_.insert(recorded_.end(), d.begin(), d.end());
+        dirty_.clear();
         for (int b : d) dirty_flag_[b] = 0;
         return d;
     }
     bool has_dirty() const { return !dirty_.empty(); }
+    // These entries of the device table may not hold the table's values: they
+    // are changed entries again.
+    void mark_dirty(const std::vector<int> &entries) {
+        for (int b : entries) mark(b);
+    }
+    // The recording is closed, kept or not: what it would update is still to
+    // do for every call that runs before it.  Returns those entries, which a
+    // replay overwrites with the recorded values (mark_dirty them then).
+    std::vector<int> end_recording() {
+        std::vector<int> r;
+        r.swap(recorded_);
+        mark_dirty(r);
+        return r;
+    }
 
     // Page copies queued by copy-on-write; clears the list.
     std::vector<Copy> take_copies() {
@@ -293,6 +313,7 @@ class KvPages {
     int live_len_ = 0;
     std::vector<int> dirty_;
     std::vector<uint8_t> dirty_flag_;
+    std::vector<int> recorded_;  // entries whose update went into the open recording
     std::vector<Copy> copies_;
     std::unordered_map<uint64_t, Entry> store_;
     std::unordered_map<int, uint64_t> phys_hash_;
