@@ -857,6 +857,14 @@ int decode_pages_per_split(int pages) {
     return pages <= 128 ? 1 : pages <= 256 ? 2 : (pages + 127) / 128;
 }
 
+// Whether the output shares memory with a row or norm vector the call reads.
+bool out_overlaps_inputs(const DecodeArgs &a) {
+    const uintptr_t o = (uintptr_t)a.out, kvn = (uintptr_t)a.kv_heads * kHeadDim * 4, on = kvn * kGroup;
+    auto meets = [&](const float *p, uintptr_t n) { return (uintptr_t)p < o + on && o < (uintptr_t)p + n; };
+    return meets(a.q, on) || meets(a.knew, kvn) || meets(a.vnew, kvn) || meets(a.qnw, kHeadDim * 4) ||
+           meets(a.knw, kHeadDim * 4);
+}
+
 hipError_t launch_decode(int kv_dtype, const DecodeArgs &args, hipStream_t s) {
     DecodeArgs a = args;
     // Work split: pages of the cached positions [0, L-1), the new token riding
@@ -873,8 +881,11 @@ hipError_t launch_decode(int kv_dtype, const DecodeArgs &args, hipStream_t s) {
     const bool full = a.rope_dim == kHeadDim;
     DecodeKernel k;
     // A short cache in one launch (pick_one): the split form's second launch
-    // and the partials' round trip cost more than the tiles' longer walk.
-    if (in_args && one_launch(kv_dtype, pages)) {
+    // and the partials' round trip cost more than the tiles' longer walk.  Its
+    // kOneSlices workgroups of a kv head all read the heads' q and each writes
+    // a slice of the output, so an output in place of an input takes the split
+    // form, which writes it once every input has been read.
+    if (in_args && one_launch(kv_dtype, pages) && !out_overlaps_inputs(a)) {
         a.nsplit = 1;
         k = kv_dtype == 0 ? pick_one<F32>(pages, full) : kv_dtype == 1 ? pick_one<F16>(pages, full) : pick_one<BF16>(pages, full);
         KernelSpan span("decode_attn", s, true);

@@ -84,3 +84,24 @@ def test_replay_keeps_its_pages(hip_available, dtype, pos):
         be.graph_destroy(g)
     finally:
         be.Dispose()
+
+
+@pytest.mark.parametrize("dtype,pos", [(F32, 150), (F16, 70), (BF16, 300), (F16, 512)])
+def test_output_in_place_of_q(hip_available, dtype, pos):
+    """out may be the q buffer: the call then writes it after every read."""
+    kb, vb = cache_rows(17, pos, salt=7)
+    q, k, v, qnw, knw = new_token(17, 7, "gamma")
+    be = HipBackend(0).configure(HQ, HKV, D, D, BASE, EPS).create_cache(1, 640, dtype)
+    try:
+        be.UploadKv(0, 0, pos, kb, vb)
+        ptrs = dev_inputs(be, [q, k, v, qnw, knw])
+        dout = be.alloc(q.nbytes)
+        outs = []
+        for d in (dout, ptrs[0]):
+            be.decode_dev(0, pos, *ptrs, d)
+            be.sync()
+            outs.append(be.download(np.empty(HQ * D, np.float32), d))
+    finally:
+        be.Dispose()
+    # two forms of the same sums: q and P enter the MFMA in 16-bit pairs
+    assert max_rel(outs[1], outs[0]) <= 1e-3
