@@ -645,10 +645,14 @@ int hymt_attn_decode_noalloc(hymt_ctx *c, int layer, int pos, const float *q, co
 // for every pair (1: unsplit), or 0 where the range is cut by a tile count
 // instead (below).  At most 256 / pairs (rounded down), so that the items are
 // one round of the chip: a workgroup holds a CU's LDS, and a few items more
-// than 256 cost a whole second round (1000 rows over 8192: 4 ns 79 us, 2 ns
-// 75 us, unsplit 112 us; 700 rows 89 -> 66 us against a cut that made 264
-// items).  The same count for every pair, because the kernels then find their
-// item in closed form instead of by a loop over the pairs.
+// than 256 cost a whole second round (700 rows over 8192: 89 -> 66 us against a
+// cut that made 264 items).  The same count for every pair, because the kernels
+// then find their item in closed form instead of by a loop over the pairs.
+//
+// From 128 pairs on a call stays whole, as a sum that is kept in fp32 to the
+// end: split items hand their outputs over in the cache type, and a split of
+// 128 pairs in two would be the only gain (1000 rows over 8192: 75 us instead
+// of 113).
 //
 // Up to 304 rows every split shortens the call and the longest is taken;
 // beyond, the partials' round trip weighs against the tiles saved.  Fitted to
@@ -658,8 +662,8 @@ int hymt_attn_decode_noalloc(hymt_ctx *c, int layer, int pos, const float *q, co
 // Over a short cache (under 48 tiles) up to 304 rows keep the cut by tiles: the
 // two differ there by less than a step.
 static int uniform_splits(int pos, int seq, int nb16, int npairs, int kv_heads, int max_tiles) {
+    if (npairs * kv_heads >= 128) return 0;
     const int most = 256 / (npairs * kv_heads);
-    if (most < 1) return 0;
     int best = 1;
     if (nb16 <= 19) {
         if (max_tiles < 48) return 0;
@@ -775,7 +779,7 @@ static int prefill_impl(hymt_ctx *c, int layer, int pos, int seq, const void *q,
             for (int b = npages; b < kArgPages; b++) f.pages[b] = f.pages[npages - 1];
         }
         // Work items: the kv range of block pairs is split when the (kv head,
-        // pair) combinations fill at most half the GPU.
+        // pair) combinations fill less than half the GPU.
         int max_tiles = 0;
         for (int pr = 0; pr < f.npairs; pr++) max_tiles = std::max(max_tiles, pair_tiles(pos, pr, f.nb16, seq));
         const int uniform_ns = uniform_splits(pos, seq, f.nb16, f.npairs, c->kv_heads, max_tiles);
