@@ -656,9 +656,15 @@ int hymt_attn_decode_noalloc(hymt_ctx *c, int layer, int pos, const float *q, co
 //
 // Up to 304 rows every split shortens the call and the longest is taken;
 // beyond, the partials' round trip weighs against the tiles saved.  Fitted to
-// 310-1020 rows over 0-8192 positions with 1-6 splits: 1.4 us per step of two
-// tiles (64 positions each) and 5 ns per row and split, e.g. 512 rows: over 0
-// 17.5 / 19.3 / 20.5 us for 1 / 2 / 4 splits, over 2048 39.7 / 30.7 / 27.2.
+// 310-1020 rows over 0-8192 positions with 1-6 splits and 4 kv heads: 1.4 us per
+// step of two tiles (64 positions each) and 5 ns per row and split, e.g. 512
+// rows: over 0 17.5 / 19.3 / 20.5 us for 1 / 2 / 4 splits, over 2048 39.7 / 30.7 /
+// 27.2.  The round trip grows with the kv heads (a row's partials are 4 heads of
+// each); below 4 the chip is emptier and it costs a little less than that.
+// us with the split count so chosen / with 5 ns at any kv head count / with the
+// cut by tiles: 1 kv head, 512 rows over 0 14.8 / 17.0 / 15.1, over 512 16.3 / 18.6 /
+// 16.3, 2048 rows over 2048 31.2 / 39.4 / 44.4; 2 kv heads, 900 rows over 2048 27.9 /
+// 29.6 / 42.7; 8 kv heads, 400 rows over 512 23.9 / 26.1 / 32.6.
 // Over a short cache (under 48 tiles) up to 304 rows keep the cut by tiles: the
 // two differ there by less than a step.
 static int uniform_splits(int pos, int seq, int nb16, int npairs, int kv_heads, int max_tiles) {
@@ -671,10 +677,11 @@ static int uniform_splits(int pos, int seq, int nb16, int npairs, int kv_heads, 
         best = (max_tiles + cap - 1) / cap;
     } else {
         const int shortest = pair_tiles(pos, npairs - 1, nb16, seq);
+        const long per20 = kv_heads >= 4 ? 5 * kv_heads : 4 * kv_heads;  // of a row and split, in 20ths of 5 ns
         long best_cost = -1;
         for (int ns = 1; ns <= std::min(most, shortest); ns++) {
             const int steps = ((max_tiles + ns - 1) / ns + 1) / 2;
-            const long cost = 280L * steps + (ns > 1 ? (long)seq * ns : 0);  // units of 5 ns
+            const long cost = 20 * 280L * steps + (ns > 1 ? per20 * seq * ns : 0);
             if (best_cost < 0 || cost < best_cost) {
                 best_cost = cost;
                 best = ns;

@@ -8,8 +8,9 @@ import numpy as np
 import pytest
 
 from hymt2sharp_amd import HipBackend
+from hymt2sharp_amd import synth as S
 from hymt2sharp_amd._native import BF16, F16, ArgumentError
-from tests.attn_cases import BASE, D, EPS
+from tests.attn_cases import BASE, D, EPS, cache_rows, new_token
 from tests.test_gpu_prefill import check, run_prefill
 
 pytestmark = pytest.mark.gpu
@@ -29,24 +30,21 @@ def test_split_rule_edges(oracle, hip_available, dtype, pos, seq):
     assert np.array_equal(vd, vref)
 
 
-@pytest.mark.parametrize("kv_heads,seq,merges", [(4, 992, 1), (4, 993, 0), (4, 1024, 0), (8, 480, 1), (8, 512, 0),
-                                                 (2, 1984, 1), (2, 2048, 0)])
-def test_128_pairs_stay_whole(hip_available, kv_heads, seq, merges):
-    """From 128 (block pair, kv head) items on a call keeps every sum in fp32
-    to its output: no partial in the cache type, no merge, and so no workspace
-    that a first call under recording would have to grow."""
-    be = HipBackend(0).configure(4 * kv_heads, kv_heads, D, D, BASE, EPS).create_cache(1, 6144 + seq, BF16)
+def merges_of(kv_heads, pos, seq, record):
+    """Merge launches of one call (1: split), after a recording of it without a
+    warm-up if `record`."""
+    be = HipBackend(0).configure(4 * kv_heads, kv_heads, D, D, BASE, EPS).create_cache(1, pos + seq, BF16)
     try:
-        be.MapRange(0, 6144 + seq)
+        be.MapRange(0, pos + seq)
         bufs = [be.alloc(n) for n in (seq * 4 * kv_heads * D * 2, seq * kv_heads * D * 2, seq * kv_heads * D * 2,
                                       seq * 4 * kv_heads * D * 4)]
         for b, n in zip(bufs, (4, 1, 1, 8)):
             be.upload(b, np.zeros(seq * n * kv_heads * D, np.uint16))
 
         def call():
-            be.prefill_dev(0, 6144, seq, *bufs[:3], BF16, None, None, bufs[3])
+            be.prefill_dev(0, pos, seq, *bufs[:3], BF16, None, None, bufs[3])
 
-        if not merges:
+        if record:
             be.graph_begin()
             call()
             be.graph_destroy(be.graph_end())
@@ -55,9 +53,51 @@ def test_128_pairs_stay_whole(hip_available, kv_heads, seq, merges):
         be.sync()
         assert be.timing("prefill_flash")[0] == 1
         try:
-            count = be.timing("prefill_merge")[0]
+            return be.timing("prefill_merge")[0]
         except ArgumentError:  # none was timed
-            count = 0
-        assert count == merges
+            return 0
     finally:
         be.Dispose()
+
+
+@pytest.mark.parametrize("kv_heads,seq,merges", [(4, 992, 1), (4, 993, 0), (4, 1024, 0), (8, 480, 1), (8, 512, 0),
+                                                 (2, 1984, 1), (2, 2048, 0)])
+def test_128_pairs_stay_whole(hip_available, kv_heads, seq, merges):
+    """From 128 (block pair, kv head) items on a call keeps every sum in fp32
+    to its output: no partial in the cache type, no merge, and so no workspace
+    that a first call under recording would have to grow."""
+    assert merges_of(kv_heads, 6144, seq, record=not merges) == merges
+
+
+@pytest.mark.parametrize("kv_heads,pos,seq,merges", [
+    (1, 0, 512, 1), (1, 512, 600, 1), (2, 0, 400, 1),  # cheap partials: split already over a short cache
+    (4, 0, 512, 0), (4, 2048, 512, 1),
+    (8, 512, 400, 0), (8, 2048, 400, 1),               # dear ones: whole a little longer
+])
+def test_splits_weigh_the_kv_heads(hip_available, kv_heads, pos, seq, merges):
+    assert merges_of(kv_heads, pos, seq, record=False) == merges
+
+
+@pytest.mark.parametrize("kv_heads", [1, 2, 8])
+@pytest.mark.parametrize("pos,seq", [(0, 512), (700, 400), (3000, 330), (3000, 200)])
+def test_other_kv_head_counts(oracle, hip_available, kv_heads, pos, seq):
+    """The first kv heads of the usual inputs, or those twice over."""
+    def cut(a, per):  # per: heads for each kv head
+        return np.ascontiguousarray(np.concatenate([a, a], 1)[:, :per * kv_heads * D])
+    kb, vb = (cut(a, 1) for a in cache_rows(18, pos))
+    q, k, v, qnw, knw = new_token(18, 0, "gamma", seq=seq)
+    q, k, v = cut(q, 4), cut(k, 1), cut(v, 1)
+    be = HipBackend(0).configure(4 * kv_heads, kv_heads, D, D, BASE, EPS).create_cache(1, pos + seq, BF16)
+    try:
+        if pos:
+            be.UploadKv(0, 0, pos, kb, vb)
+        got = be.PrefillAttention(0, pos, q, k, v, qnw, knw)
+    finally:
+        be.Dispose()
+    caches = []
+    for b in (kb, vb):
+        caches.append(oracle.new_cache(pos + seq, kv_heads, D, BF16))
+        caches[-1][:pos] = oracle.to_storage(S.bf16_bits_to_f32(b), BF16)
+    ref = oracle.prefill_attention(q, k, v, qnw, knw, *caches, BF16, 4 * kv_heads, kv_heads, D, BASE, EPS, pos,
+                                   threads=8)
+    check(got, ref, oracle.from_storage(caches[1], BF16), BF16)
