@@ -486,8 +486,9 @@ __global__ __launch_bounds__(256) void embed_kernel(WeightDev w, int row, float 
 //    c over the four low-code sub-blocks 2 g and, from the other two MFMAs, the
 //    high-code ones 2 g + 1, and weighs them by the 6-bit scales in integers
 //    (below 2^25 together).
-// The minima take fp32 sums of x' per sub-block (which also carry an infinity
-// or NaN of x' into the result).  What is rounded is fp32 and per super-block;
+// The minima take fp32 sums of x' per sub-block.  A super-block with an infinity
+// or NaN in x' takes fp32 products instead (plain_dot), which carry it into
+// the result as the codes, scales and minima have it.  What is rounded is fp32 and per super-block;
 // x' itself is off by 2^-31 of the largest value at most, which after 256 of
 // them is below the rounding of a sum that holds the largest.  rms error over
 // 2048 rows, of the rms of y, here and in the VALU form (2048 to 8192
@@ -500,8 +501,7 @@ __global__ __launch_bounds__(256) void embed_kernel(WeightDev w, int row, float 
 // bits stored with 32's flipped, so that two masks and an or make four), each
 // MFMA's lane groups hold one 16-value sub-block each, so a lane (p, c) receives
 // digit p's sums of row c over four of them and weighs them by their signed
-// scales (below 2^29 together).  There are no minima: an infinity or NaN of x'
-// makes the digits' weight NaN.  rms error as above: normal
+// scales (below 2^29 together).  There are no minima.  rms error as above: normal
 // x 0.7e-7 to 0.9e-7 (1.5e-7 to 2.0e-7), outliers 0.8e-7 to 0.9e-7 (1.1e-7 to
 // 1.3e-7), log-normal 0.7e-7 to 0.9e-7 (1.3e-7), all positive 0.7e-7 (1.1e-7 to
 // 1.7e-7).
@@ -545,13 +545,75 @@ __device__ __forceinline__ void wave_order() {
     __builtin_amdgcn_wave_barrier();
 }
 
+// Columns 64 grp + [0, 64) of a tile's row r times x, in fp32, a code and a
+// value at a time as the VALU form has them.  Loops, not registers: this is
+// the way of super-blocks whose x' has no digits.
+template <int T> __device__ __forceinline__ float plain_dot(const uint8_t *tile, int r, int grp, const float *x) {
+    const uint32_t *q = (const uint32_t *)(tile + 16 * (16 * grp + r));  // piece m's dword j: q[256 m + j]
+    float y = 0.f;
+    if constexpr (T == kW_Q4_K) {  // sub-blocks 2 grp (low codes) and 2 grp + 1
+        const uint8_t *sm = tile + kQ4Scales + 16 * r + 4 * grp;
+        const uint32_t dd = *(const uint32_t *)(tile + kQ4D + 4 * r);
+#pragma unroll 1
+        for (int h = 0; h < 2; h++) {
+            float a = 0.f, sx = 0.f;
+#pragma unroll 1
+            for (int j = 0; j < 8; j++) {
+                const uint32_t k = q[256 * (j >> 2) + (j & 3)] >> (4 * h);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float v = x[32 * h + 4 * j + e];
+                    a = fmaf((float)((k >> (8 * e)) & 0xFu), v, a);
+                    sx += v;
+                }
+            }
+            y += h2f(dd & 0xFFFF) * ((float)sm[h] * a) - h2f(dd >> 16) * ((float)sm[2 + h] * sx);
+        }
+    } else if constexpr (T == kW_Q6_K) {  // sub-blocks 4 grp + m
+        const uint32_t *hi = (const uint32_t *)(tile + kQ6Hi + 16 * (16 * grp + r));
+        const int8_t *sc = (const int8_t *)(tile + kQ6Scales + 16 * r + 4 * grp);
+#pragma unroll 1
+        for (int m = 0; m < 4; m++) {
+            float a = 0.f, sx = 0.f;
+#pragma unroll 1
+            for (int j = 0; j < 4; j++) {
+                const uint32_t lo = q[256 * (m >> 1) + j] >> (4 * (m & 1)), hb = hi[j] >> (6 - 2 * m);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {  // the stored upper bit is flipped
+                    const uint32_t k = ((lo >> (8 * e)) & 0xFu) | ((((hb >> (8 * e)) & 3u) ^ 2u) << 4);
+                    const float v = x[16 * m + 4 * j + e];
+                    a = fmaf((float)k, v, a);
+                    sx += v;
+                }
+            }
+            y += (float)sc[m] * (a - 32.f * sx);
+        }
+        y *= h2f(*(const uint16_t *)(tile + kQ6D + 2 * r));
+    } else {  // blocks 2 grp, 2 grp + 1
+        const uint16_t *d = (const uint16_t *)(tile + kQ8D + 16 * r + 4 * grp);
+#pragma unroll 1
+        for (int h = 0; h < 2; h++) {
+            float a = 0.f;
+#pragma unroll 1
+            for (int j = 0; j < 8; j++) {
+                const uint32_t k = q[256 * (2 * h + (j >> 2)) + (j & 3)];
+#pragma unroll
+                for (int e = 0; e < 4; e++) a = fmaf((float)(int8_t)(k >> (8 * e)), x[32 * h + 4 * j + e], a);
+            }
+            y += h2f(d[h]) * a;
+        }
+    }
+    return y;
+}
+
 template <int T, int RT, int NW, int NSB, int MODE>
 __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const float *__restrict__ xg,
                                                           float *__restrict__ y, int flags,
                                                           const float *__restrict__ nw, float eps) {
     constexpr bool Q6 = T == kW_Q6_K, Q8 = T == kW_Q8_0;
     constexpr int kTile = Q8 ? kQ8Tile : Q6 ? kQ6Tile : kQ4Tile;
-    // a wave's super-blocks as digits, [group][digit][64 columns], and zeros
+    // a wave's super-blocks as digits, [group][digit][64 columns], or as they
+    // are (the bits of `plain`), and zeros
     __shared__ __attribute__((aligned(16))) uint8_t s_x[NW][NSB + 1][1024];
     __shared__ float s_p[NW][RT][16];
     __shared__ float s_ss[NW];
@@ -573,12 +635,15 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
     // rows and the same rows of up, or (RT = 1) a tile is 8 of each
     uint4 q0[RT][NSB], q1[RT][NSB], q2[RT][NSB], q3[RT][NSB], sm[RT][NSB];
     uint32_t dd[RT][NSB];
+    auto row_of = [&](int i) {
+        return min(out_swiglu && RT == 1 ? (c >> 3) * F + 8 * (int)blockIdx.x + (c & 7)
+                   : out_swiglu          ? (i & 1) * F + 16 * ((int)(blockIdx.x * RT + i) >> 1) + c
+                                         : 16 * (int)(blockIdx.x * RT + i) + c,
+                   w.rows - 1);
+    };
 #pragma unroll
     for (int i = 0; i < RT; i++) {
-        const int row = min(out_swiglu && RT == 1 ? (c >> 3) * F + 8 * (int)blockIdx.x + (c & 7)
-                            : out_swiglu          ? (i & 1) * F + 16 * ((int)(blockIdx.x * RT + i) >> 1) + c
-                                                  : 16 * (int)(blockIdx.x * RT + i) + c,
-                            w.rows - 1);
+        const int row = row_of(i);
         const int r = row & 15, li = grp * 16 + r;
         const uint8_t *b = (const uint8_t *)w.q + ((size_t)(row >> 4) * nsb + sb0) * kTile;
 #pragma unroll
@@ -604,6 +669,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
 
     if (lane < 16) *(uint32_t *)(s_x[wave][NSB] + 4 * lane) = 0;
     float S0[NSB], S1[NSB], wgt[NSB], ss = 0.f;
+    uint32_t plain = 0;
 #pragma unroll
     for (int s = 0; s < NSB; s++) {
         float v[4] = {xv[s].x, xv[s].y, xv[s].z, xv[s].w};
@@ -639,7 +705,12 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
         const int e = min(max((int)(mx >> 23), 30), 254);
         const float sc = __uint_as_float((uint32_t)(283 - e) << 23);
         wgt[s] = __uint_as_float((uint32_t)(e - 29 + 8 * grp) << 23);  // of digit `grp`
-        if ((Q6 || Q8) && mx >= 0x7F800000u) wgt[s] = NAN;
+        if (__builtin_amdgcn_readfirstlane(mx) >= 0x7F800000u) {  // an infinity or NaN: no digits
+            plain |= 1u << s;
+            wgt[s] = S0[s] = S1[s] = 0.f;
+            *(float4 *)(s_x[wave][s] + 16 * lane) = make_float4(v[0], v[1], v[2], v[3]);
+            continue;
+        }
         // four signed digits of each column: with 0x80 added to the lower
         // three bytes they are the bytes less 0x80
         uint32_t t[4];
@@ -722,6 +793,18 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
             const float m0 = (float)((kg >> 16) & 0xFFu), m1 = (float)(kg >> 24);
             acc[i] = fmaf(d, (float)t * wgt[s], acc[i]);
             acc[i] = fmaf(-dmin, fmaf(m0, S0[s], m1 * S1[s]), acc[i]);
+        }
+    }
+    if (plain) {
+#pragma unroll 1
+        for (uint32_t left = plain; left; left &= left - 1) {
+            const int s = __builtin_ctz(left);
+#pragma unroll
+            for (int i = 0; i < RT; i++) {
+                const int row = row_of(i);
+                const uint8_t *b = (const uint8_t *)w.q + ((size_t)(row >> 4) * nsb + sb0 + s) * kTile;
+                acc[i] += plain_dot<T>(b, row & 15, grp, (const float *)s_x[wave][s] + 64 * grp);
+            }
         }
     }
 #pragma unroll

@@ -1,0 +1,75 @@
+"""What the matrix-core GEMVs (hymt2sharp_amd/csrc/gemv.hip, gemv_kq_kernel) make
+of inputs whose values lie far apart: infinities and NaN."""
+import numpy as np
+import pytest
+
+from hymt2sharp_amd import HipBackend
+from hymt2sharp_amd import _native as N
+from hymt2sharp_amd import synth as S
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [N.W_Q4_K, N.W_Q6_K, N.W_Q8_0]
+
+
+def weights(wtype, seed, rows, cols, zero=()):
+    """A random matrix and its fp64 values; the columns `zero` have weight 0 in
+    every row (for Q4_K their super-blocks have no minima)."""
+    raw = np.frombuffer(S.random_weight(seed, wtype, rows, cols), np.uint8).copy()
+    size = {N.W_Q4_K: 144, N.W_Q6_K: 210, N.W_Q8_0: 34 * 8}[wtype]
+    b = raw.reshape(rows, cols // 256, size)
+    for col in zero:
+        sb, j = divmod(col, 256)
+        if wtype == N.W_Q8_0:
+            b[:, sb, 34 * (j // 32) + 2 + j % 32] = 0
+        elif wtype == N.W_Q4_K:
+            b[:, sb, 2:4] = 0
+            b[:, sb, 16 + 32 * (j // 64) + j % 32] &= 0x0F if j % 64 >= 32 else 0xF0
+        else:  # code 32: low bits 0, high bits 2
+            n, quarter, l = j // 128, j % 128 // 32, j % 32
+            b[:, sb, 64 * n + 32 * (quarter & 1) + l] &= 0x0F if quarter >= 2 else 0xF0
+            h = b[:, sb, 128 + 32 * n + l]
+            b[:, sb, 128 + 32 * n + l] = (h & ~np.uint8(3 << 2 * quarter)) | np.uint8(2 << 2 * quarter)
+    raw = raw.tobytes()
+    W = O.dequant(wtype, raw, rows, cols).astype(np.float64)
+    assert not W[:, list(zero)].any()
+    return raw, W
+
+
+def gemv(wtype, raw, rows, cols, x, **kw):
+    outs = rows // 2 if kw.get("swiglu_out") else rows
+    be = HipBackend(0)
+    try:
+        w = be.weight_upload(wtype, rows, cols, raw)
+        dx, dy, dg = be.alloc(4 * x.size), be.alloc(4 * outs), None
+        be.upload(dx, x)
+        be.upload(dy, np.zeros(outs, np.float32))
+        if "gamma" in kw:
+            dg = be.alloc(4 * cols)
+            be.upload(dg, kw.pop("gamma"))
+        be.gemv(w, dx, dy, rmsnorm=dg, eps=1e-6, **kw)
+        be.sync()
+        return be.download(np.empty(outs, np.float32), dy)
+    finally:
+        be.Dispose()
+
+
+@pytest.mark.parametrize("rows,cols", [(33, 2048), (8208, 2048), (20, 8192)])
+@pytest.mark.parametrize("bad", [{777: np.inf}, {5: -np.inf}, {300: np.inf, 1999: np.inf}, {300: np.inf, 301: -np.inf},
+                                 {0: np.nan}])
+@pytest.mark.parametrize("wtype", TYPES)
+def test_infinities_and_nan(hip_available, wtype, bad, rows, cols):
+    """As the products have it: Q8_0's are code times value, Q4_K's and Q6_K's
+    take an offset off afterwards, where infinity less infinity is NaN.  The
+    rows' other super-blocks do not hide it."""
+    raw, W = weights(wtype, 12, rows, cols)
+    x = np.random.default_rng(3).standard_normal(cols).astype(np.float32)
+    for c, v in bad.items():
+        x[c] = v
+    y = gemv(wtype, raw, rows, cols, x)
+    with np.errstate(invalid="ignore"):
+        want = W @ x.astype(np.float64) if wtype == N.W_Q8_0 else np.full(rows, np.nan)
+    assert np.array_equal(y.astype(np.float64), want, equal_nan=True)
+    if wtype == N.W_Q8_0 and len(bad) == 1:
+        assert np.isinf(y).any() or np.isnan(x).any()
