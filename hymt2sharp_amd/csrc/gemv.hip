@@ -476,21 +476,23 @@ __global__ __launch_bounds__(256) void embed_kernel(WeightDev w, int row, float 
 // where the bytes take 25.  Here a super-block's 256 products run on
 // v_mfma_i32_16x16x64_i8, exactly:
 //  - the codes enter as they are, bytes of 0..15 (one mask per four weights);
-//  - x' enters as a 31-bit fixed-point number in four signed bytes, x' s =
-//    sum_p d_p 256^p, s the power of two that brings the super-block's largest
-//    |x'| to [2^29, 2^30): at least fp32's 24 bits of every value within 2^-6
-//    of the largest, and 2^-30 of the largest for the rest;
+//  - x' enters as a 61-bit fixed-point number, x' s = h + l 2^-30, h and l in
+//    four signed bytes each, sum_p d_p 256^p; s is the power of two that brings
+//    the super-block's largest |x'| to [2^29, 2^30).  That holds every fp32
+//    value down to 2^-36 of the largest exactly.  A super-block with smaller
+//    ones (but 0), an infinity or NaN takes fp32 products instead (plain_dot).
+//    h alone lost what lay 2^-30 below the largest: beside a value 3000 times
+//    the others, at weight 0, the error was 2.1e-6 (1.2e-7 with l); l costs a
+//    second set of products, 2-8 % of a call (three layers' worth of Q4_K GEMVs
+//    1 %, 120818 x 2048 25.3 -> 28.3 us; Q8_0 there 47.4 -> 44.5).
 //  - the A operand's 16 rows are (digit p, sub-block pair g): row 4 p + g holds
-//    digit p of x' in the k range of lane group g and zeros elsewhere, its 16
+//    digit p of h (or l) in the k range of lane group g and zeros elsewhere, its 16
 //    columns are weight rows.  So a lane (p, c) receives digit p's sums of row
 //    c over the four low-code sub-blocks 2 g and, from the other two MFMAs, the
 //    high-code ones 2 g + 1, and weighs them by the 6-bit scales in integers
 //    (below 2^25 together).
-// The minima take fp32 sums of x' per sub-block.  A super-block with an infinity
-// or NaN in x' takes fp32 products instead (plain_dot), which carry it into
-// the result as the codes, scales and minima have it.  What is rounded is fp32 and per super-block;
-// x' itself is off by 2^-31 of the largest value at most, which after 256 of
-// them is below the rounding of a sum that holds the largest.  rms error over
+// The minima take fp32 sums of x' per sub-block.  What is rounded is fp32 and per
+// super-block.  rms error over
 // 2048 rows, of the rms of y, here and in the VALU form (2048 to 8192
 // columns): normal x 0.7e-7 to 1.1e-7 (0.9e-7 to 1.4e-7), one value per
 // super-block 100 to 30000 times the others 0.8e-7 to 1.0e-7 (1.1e-7 to
@@ -582,11 +584,13 @@ template <int T> __device__ __forceinline__ float plain_dot(const uint8_t *tile,
                 for (int e = 0; e < 4; e++) {  // the stored upper bit is flipped
                     const uint32_t k = ((lo >> (8 * e)) & 0xFu) | ((((hb >> (8 * e)) & 3u) ^ 2u) << 4);
                     const float v = x[16 * m + 4 * j + e];
-                    a = fmaf((float)k, v, a);
+                    a = fmaf((float)(int)(k - 32u), v, a);
                     sx += v;
                 }
             }
-            y += (float)sc[m] * (a - 32.f * sx);
+            // with the offset taken off afterwards (code v less 32 v) an
+            // infinity of x' is NaN whatever the code: 0 sx keeps that
+            y += (float)sc[m] * fmaf(0.f, sx, a);
         }
         y *= h2f(*(const uint16_t *)(tile + kQ6D + 2 * r));
     } else {  // blocks 2 grp, 2 grp + 1
@@ -612,9 +616,10 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
                                                           const float *__restrict__ nw, float eps) {
     constexpr bool Q6 = T == kW_Q6_K, Q8 = T == kW_Q8_0;
     constexpr int kTile = Q8 ? kQ8Tile : Q6 ? kQ6Tile : kQ4Tile;
-    // a wave's super-blocks as digits, [group][digit][64 columns], or as they
-    // are (the bits of `plain`), and zeros
-    __shared__ __attribute__((aligned(16))) uint8_t s_x[NW][NSB + 1][1024];
+    // a wave's super-blocks as digits, [first, second][group][digit][64
+    // columns], or as they are (the bits of `plain`), and zeros
+    __shared__ __attribute__((aligned(16))) uint8_t s_x[NW][NSB][2][1024];
+    __shared__ __attribute__((aligned(16))) uint8_t s_zero[NW][64];
     __shared__ float s_p[NW][RT][16];
     __shared__ float s_ss[NW];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -667,7 +672,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
     // nothing moves across: the weight loads stay ahead of the first wait on x
     __builtin_amdgcn_sched_barrier(0);
 
-    if (lane < 16) *(uint32_t *)(s_x[wave][NSB] + 4 * lane) = 0;
+    if (lane < 16) *(uint32_t *)(s_zero[wave] + 4 * lane) = 0;
     float S0[NSB], S1[NSB], wgt[NSB], ss = 0.f;
     uint32_t plain = 0;
 #pragma unroll
@@ -705,25 +710,40 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
         const int e = min(max((int)(mx >> 23), 30), 254);
         const float sc = __uint_as_float((uint32_t)(283 - e) << 23);
         wgt[s] = __uint_as_float((uint32_t)(e - 29 + 8 * grp) << 23);  // of digit `grp`
-        if (__builtin_amdgcn_readfirstlane(mx) >= 0x7F800000u) {  // an infinity or NaN: no digits
+        // x' 2^k = h + l 2^-30, each 30 bits and a sign; what is then left is
+        // of values below 2^-36 of the largest, or an infinity or NaN
+        int t[2][4];
+        bool left = false;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float u = v[j] * sc;
+            t[0][j] = (int)u;
+            const float r = (u - (float)t[0][j]) * 1073741824.f;
+            t[1][j] = (int)r;
+            left |= r != (float)t[1][j];
+        }
+        if (__ballot(left)) {  // no digits: plain_dot takes the super-block
             plain |= 1u << s;
             wgt[s] = S0[s] = S1[s] = 0.f;
-            *(float4 *)(s_x[wave][s] + 16 * lane) = make_float4(v[0], v[1], v[2], v[3]);
+            *(float4 *)(s_x[wave][s][0] + 16 * lane) = make_float4(v[0], v[1], v[2], v[3]);
             continue;
         }
-        // four signed digits of each column: with 0x80 added to the lower
-        // three bytes they are the bytes less 0x80
-        uint32_t t[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) t[j] = ((uint32_t)(int)(v[j] * sc) + 0x00808080u) ^ 0x00808080u;
-        // digit p of the 4 columns as one dword
-        const uint32_t a0 = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u), a1 = __builtin_amdgcn_perm(t[1], t[0], 0x07030602u);
-        const uint32_t b0 = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u), b1 = __builtin_amdgcn_perm(t[3], t[2], 0x07030602u);
-        uint32_t *p = (uint32_t *)(s_x[wave][s] + grp * 256 + 4 * (lane & 15));
-        p[0] = __builtin_amdgcn_perm(b0, a0, 0x05040100u);
-        p[16] = __builtin_amdgcn_perm(b0, a0, 0x07060302u);
-        p[32] = __builtin_amdgcn_perm(b1, a1, 0x05040100u);
-        p[48] = __builtin_amdgcn_perm(b1, a1, 0x07060302u);
+        for (int d = 0; d < 2; d++) {
+            // four signed digits of each column: with 0x80 added to the lower
+            // three bytes they are the bytes less 0x80
+            uint32_t b[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) b[j] = ((uint32_t)t[d][j] + 0x00808080u) ^ 0x00808080u;
+            // digit p of the 4 columns as one dword
+            const uint32_t a0 = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u), a1 = __builtin_amdgcn_perm(b[1], b[0], 0x07030602u);
+            const uint32_t b0 = __builtin_amdgcn_perm(b[3], b[2], 0x05010400u), b1 = __builtin_amdgcn_perm(b[3], b[2], 0x07030602u);
+            uint32_t *p = (uint32_t *)(s_x[wave][s][d] + grp * 256 + 4 * (lane & 15));
+            p[0] = __builtin_amdgcn_perm(b0, a0, 0x05040100u);
+            p[16] = __builtin_amdgcn_perm(b0, a0, 0x07060302u);
+            p[32] = __builtin_amdgcn_perm(b1, a1, 0x05040100u);
+            p[48] = __builtin_amdgcn_perm(b1, a1, 0x07060302u);
+        }
     }
     wave_order();
     float acc[RT] = {};
@@ -731,8 +751,13 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
     const int zoff = (c & 3) == grp ? grp * 256 + (c >> 2) * 64 : -1;
 #pragma unroll
     for (int s = 0; s < NSB; s++) {
-        const i32x4 *xp = (const i32x4 *)(zoff < 0 ? s_x[wave][NSB] : s_x[wave][s] + zoff);
-        const i32x4 xa[4] = {xp[0], xp[1], xp[2], xp[3]};  // Q4_K: low codes' columns, high codes'
+        i32x4 xa[2][4];  // Q4_K: low codes' columns, high codes'
+#pragma unroll
+        for (int d = 0; d < 2; d++) {
+            const i32x4 *xp = (const i32x4 *)(zoff < 0 ? s_zero[wave] : s_x[wave][s][d] + zoff);
+#pragma unroll
+            for (int m = 0; m < 4; m++) xa[d][m] = xp[m];
+        }
 #pragma unroll
         for (int i = 0; i < RT; i++) {
             const uint4 a = q0[i][s], b = q1[i][s];
@@ -741,24 +766,28 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
                 const uint4 e = q2[i][s], f = q3[i][s];
                 const i32x4 l0 = {(int)a.x, (int)a.y, (int)a.z, (int)a.w}, l1 = {(int)b.x, (int)b.y, (int)b.z, (int)b.w};
                 const i32x4 h0 = {(int)e.x, (int)e.y, (int)e.z, (int)e.w}, h1 = {(int)f.x, (int)f.y, (int)f.z, (int)f.w};
-                i32x4 L = {0, 0, 0, 0}, H = {0, 0, 0, 0};
-                L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[0], l0, L, 0, 0, 0);
-                H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[2], h0, H, 0, 0, 0);
-                L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[1], l1, L, 0, 0, 0);
-                H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[3], h1, H, 0, 0, 0);
-                float t = 0.f;
+                float t[2];
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    t = fmaf(h2f(k[g] & 0xFFFF), (float)L[g], t);
-                    t = fmaf(h2f(k[g] >> 16), (float)H[g], t);
+                for (int d = 0; d < 2; d++) {
+                    i32x4 L = {0, 0, 0, 0}, H = {0, 0, 0, 0};
+                    L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[d][0], l0, L, 0, 0, 0);
+                    H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[d][2], h0, H, 0, 0, 0);
+                    L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[d][1], l1, L, 0, 0, 0);
+                    H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[d][3], h1, H, 0, 0, 0);
+                    t[d] = 0.f;
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        t[d] = fmaf(h2f(k[g] & 0xFFFF), (float)L[g], t[d]);
+                        t[d] = fmaf(h2f(k[g] >> 16), (float)H[g], t[d]);
+                    }
                 }
-                acc[i] = fmaf(t, wgt[s], acc[i]);
+                acc[i] = fmaf(fmaf(t[1], 0x1p-30f, t[0]), wgt[s], acc[i]);
                 continue;
             }
             if constexpr (Q6) {
                 const uint32_t h[4] = {q2[i][s].x, q2[i][s].y, q2[i][s].z, q2[i][s].w};
                 const uint32_t lo[2][4] = {{a.x, a.y, a.z, a.w}, {b.x, b.y, b.z, b.w}};
-                int t = 0;
+                int t[2] = {0, 0};
 #pragma unroll
                 for (int m = 0; m < 4; m++) {  // columns 64 g + 16 m + [0, 16): sub-block 4 g + m
                     i32x4 f;
@@ -767,11 +796,14 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
                         const uint32_t l = m & 1 ? lo[m >> 1][j] >> 2 : lo[m >> 1][j] << 2;
                         f[j] = (int)(((h[j] << (2 * m)) & 0xC0C0C0C0u) | (l & 0x3C3C3C3Cu));
                     }
-                    const i32x4 D = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[m], f, i32x4{0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
-                    for (int g = 0; g < 4; g++) t += __mul24((int)(int8_t)(k[g] >> (8 * m)), D[g]);
+                    for (int d = 0; d < 2; d++) {
+                        const i32x4 D = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[d][m], f, i32x4{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+                        for (int g = 0; g < 4; g++) t[d] += __mul24((int)(int8_t)(k[g] >> (8 * m)), D[g]);
+                    }
                 }
-                acc[i] = fmaf(h2f(dd[i][s]), (float)t * 0.25f * wgt[s], acc[i]);
+                acc[i] = fmaf(h2f(dd[i][s]), fmaf((float)t[1], 0x1p-30f, (float)t[0]) * 0.25f * wgt[s], acc[i]);
                 continue;
             }
             constexpr uint32_t M = 0x0F0F0F0Fu;
@@ -779,19 +811,22 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
             const i32x4 l1 = {(int)(b.x & M), (int)(b.y & M), (int)(b.z & M), (int)(b.w & M)};
             const i32x4 h0 = {(int)((a.x >> 4) & M), (int)((a.y >> 4) & M), (int)((a.z >> 4) & M), (int)((a.w >> 4) & M)};
             const i32x4 h1 = {(int)((b.x >> 4) & M), (int)((b.y >> 4) & M), (int)((b.z >> 4) & M), (int)((b.w >> 4) & M)};
-            i32x4 L = {0, 0, 0, 0}, H = {0, 0, 0, 0};
-            L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[0], l0, L, 0, 0, 0);
-            H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[2], h0, H, 0, 0, 0);
-            L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[1], l1, L, 0, 0, 0);
-            H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[3], h1, H, 0, 0, 0);
-            int t = 0;
+            int t[2] = {0, 0};
 #pragma unroll
-            for (int g = 0; g < 4; g++)
-                t += __mul24((int)(k[g] & 0xFFu), L[g]) + __mul24((int)((k[g] >> 8) & 0xFFu), H[g]);
+            for (int d = 0; d < 2; d++) {
+                i32x4 L = {0, 0, 0, 0}, H = {0, 0, 0, 0};
+                L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[d][0], l0, L, 0, 0, 0);
+                H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[d][2], h0, H, 0, 0, 0);
+                L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[d][1], l1, L, 0, 0, 0);
+                H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[d][3], h1, H, 0, 0, 0);
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    t[d] += __mul24((int)(k[g] & 0xFFu), L[g]) + __mul24((int)((k[g] >> 8) & 0xFFu), H[g]);
+            }
             const float d = h2f(dd[i][s] & 0xFFFF), dmin = h2f(dd[i][s] >> 16);
             const uint32_t kg = grp & 2 ? (grp & 1 ? k[3] : k[2]) : (grp & 1 ? k[1] : k[0]);
             const float m0 = (float)((kg >> 16) & 0xFFu), m1 = (float)(kg >> 24);
-            acc[i] = fmaf(d, (float)t * wgt[s], acc[i]);
+            acc[i] = fmaf(d, fmaf((float)t[1], 0x1p-30f, (float)t[0]) * wgt[s], acc[i]);
             acc[i] = fmaf(-dmin, fmaf(m0, S0[s], m1 * S1[s]), acc[i]);
         }
     }
@@ -803,7 +838,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
             for (int i = 0; i < RT; i++) {
                 const int row = row_of(i);
                 const uint8_t *b = (const uint8_t *)w.q + ((size_t)(row >> 4) * nsb + sb0 + s) * kTile;
-                acc[i] += plain_dot<T>(b, row & 15, grp, (const float *)s_x[wave][s] + 64 * grp);
+                acc[i] += plain_dot<T>(b, row & 15, grp, (const float *)s_x[wave][s][0] + 64 * grp);
             }
         }
     }

@@ -1,5 +1,11 @@
 """What the matrix-core GEMVs (hymt2sharp_amd/csrc/gemv.hip, gemv_kq_kernel) make
-of inputs whose values lie far apart: infinities and NaN."""
+of inputs whose values lie far apart: infinities and NaN, and values far below
+their super-block's largest, which lose nothing to it.
+
+Bound of the finite ones, root mean square over the rows: 2e-7 of the root mean
+square of y, about 3.4 roundings of 2^-24.  fp32 products added in fp32 make
+1.2e-7 to 1.6e-7 of these inputs; digits that ended 2^-30 below the largest value
+made 2e-6 and more where the largest meets zero weights."""
 import numpy as np
 import pytest
 
@@ -73,3 +79,61 @@ def test_infinities_and_nan(hip_available, wtype, bad, rows, cols):
     assert np.array_equal(y.astype(np.float64), want, equal_nan=True)
     if wtype == N.W_Q8_0 and len(bad) == 1:
         assert np.isinf(y).any() or np.isnan(x).any()
+
+
+def rms(a):
+    return float(np.sqrt(np.mean(np.square(a))))
+
+
+def check(y, ref):
+    err = rms(y.astype(np.float64) - ref) / rms(ref)
+    assert err <= 2e-7
+
+
+@pytest.mark.parametrize("factor", [3e3, 3e4, 1e6, 1e9, 1e12, 1e30])
+@pytest.mark.parametrize("wtype", TYPES)
+def test_small_values_beside_large_ones(hip_available, wtype, factor):
+    """One large value in each super-block, where every weight is 0: the rest is
+    what is left.  From 2^36 on it is what takes the products out of integers."""
+    cols = 2048
+    big = list(range(7, cols, 256))
+    raw, W = weights(wtype, 14, 512, cols, big)
+    x = np.random.default_rng(5).standard_normal(cols).astype(np.float32)
+    x[big] *= np.float32(factor)
+    check(gemv(wtype, raw, 512, cols, x), W @ x.astype(np.float64))
+
+
+@pytest.mark.parametrize("cols,mode", [(2048, ""), (6144, ""), (8192, ""), (2048, "norm"), (4096, "swiglu")])
+@pytest.mark.parametrize("wtype", TYPES)
+def test_magnitudes_all_over(hip_available, wtype, cols, mode):
+    """exp(8 N(0, 1)): within a super-block values span 2^60 and more, so some
+    take each way; every 50th value is 0."""
+    rng = np.random.default_rng(cols)
+    x = (rng.choice([-1, 1], 2 * cols) * np.exp(8 * rng.standard_normal(2 * cols)) * 1e-6).astype(np.float32)
+    x[::50] = 0
+    x[cols:2 * cols:3] = 1
+    raw, W = weights(wtype, 15, 512, cols)
+    xd = x.astype(np.float64)
+    if mode == "swiglu":
+        x[:cols] = np.clip(x[:cols], -60, 60)
+        xd = x.astype(np.float64)
+        xd = xd[:cols] / (1 + np.exp(-xd[:cols])) * xd[cols:]
+        # the sigmoid's own roundings, on every x': 1e-6 of it
+        y = gemv(wtype, raw, 512, cols, x, swiglu=True).astype(np.float64)
+        assert np.all(np.abs(y - W @ xd) <= 2e-6 * (np.abs(W) @ np.abs(xd)))
+    elif mode == "norm":
+        g = rng.uniform(0.9, 1.1, cols).astype(np.float32)
+        y = gemv(wtype, raw, 512, cols, x[:cols], gamma=g)
+        check(y, W @ (xd[:cols] / np.sqrt(np.mean(xd[:cols] ** 2) + 1e-6) * g))
+    else:
+        check(gemv(wtype, raw, 512, cols, x[:cols]), W @ xd[:cols])
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e-34, 1e-36])
+@pytest.mark.parametrize("wtype", TYPES)
+def test_tiny_values(hip_available, wtype, scale):
+    raw, W = weights(wtype, 16, 512, 2048)
+    x = (np.random.default_rng(6).standard_normal(2048) * scale).astype(np.float32)
+    y = gemv(wtype, raw, 512, 2048, x)
+    assert np.any(y != 0)
+    check(y, W @ x.astype(np.float64))
