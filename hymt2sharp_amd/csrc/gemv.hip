@@ -705,7 +705,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
         mx = max(mx, dpp<0x4E>(mx));
         mx = max(mx, dpp<0x141>(mx));
         mx = max(mx, dpp<0x140>(mx));
-        mx = rows_max(mx);
+        mx = __builtin_amdgcn_readfirstlane(rows_max(mx));
         // 2^k with mx 2^k in [2^29, 2^30), both it and its inverse normal
         const int e = min(max((int)(mx >> 23), 30), 254);
         const float sc = __uint_as_float((uint32_t)(283 - e) << 23);
@@ -721,6 +721,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
             const float r = (u - (float)t[0][j]) * 1073741824.f;
             t[1][j] = (int)r;
             left |= r != (float)t[1][j];
+            if (e > 156) left |= u == 0.f && v[j] != 0.f;  // s is below 1: the product underflowed
         }
         if (__ballot(left)) {  // no digits: plain_dot takes the super-block
             plain |= 1u << s;

@@ -90,16 +90,19 @@ def check(y, ref):
     assert err <= 2e-7
 
 
-@pytest.mark.parametrize("factor", [3e3, 3e4, 1e6, 1e9, 1e12, 1e30])
+@pytest.mark.parametrize("scale,factor", [(1, 3e3), (1, 3e4), (1, 1e6), (1, 1e9), (1, 1e12), (1, 1e30), (1e20, 1e9),
+                                          (1e-4, 1e38), (1e-20, 1e38), (1e-22, 1e57)])
 @pytest.mark.parametrize("wtype", TYPES)
-def test_small_values_beside_large_ones(hip_available, wtype, factor):
+def test_small_values_beside_large_ones(hip_available, wtype, scale, factor):
     """One large value in each super-block, where every weight is 0: the rest is
-    what is left.  From 2^36 on it is what takes the products out of integers."""
+    what is left.  From 2^36 on it is what takes the products out of integers;
+    the last are 0 at the large value's scale."""
     cols = 2048
     big = list(range(7, cols, 256))
     raw, W = weights(wtype, 14, 512, cols, big)
-    x = np.random.default_rng(5).standard_normal(cols).astype(np.float32)
-    x[big] *= np.float32(factor)
+    x = np.random.default_rng(5).standard_normal(cols) * scale
+    x[big] = scale * factor
+    x = x.astype(np.float32)
     check(gemv(wtype, raw, 512, cols, x), W @ x.astype(np.float64))
 
 
