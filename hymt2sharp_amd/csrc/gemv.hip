@@ -491,29 +491,30 @@ __global__ __launch_bounds__(256) void embed_kernel(WeightDev w, int row, float 
 //    c over the four low-code sub-blocks 2 g and, from the other two MFMAs, the
 //    high-code ones 2 g + 1, and weighs them by the 6-bit scales in integers
 //    (below 2^25 together).
-// The minima take fp32 sums of x' per sub-block.  What is rounded is fp32 and per
-// super-block.  rms error over
-// 2048 rows, of the rms of y, here and in the VALU form (2048 to 8192
-// columns): normal x 0.7e-7 to 1.1e-7 (0.9e-7 to 1.4e-7), one value per
-// super-block 100 to 30000 times the others 0.8e-7 to 1.0e-7 (1.1e-7 to
-// 1.3e-7), log-normal magnitudes with sigma 3 0.7e-7 to 0.9e-7 (0.9e-7 to
-// 1.1e-7), all x positive 0.5e-7 to 0.7e-7 (0.4e-7).
+// The minima take sums of x' per sub-block, in fp64, and a wave's products and
+// minima are summed in fp64, because they cancel: with weights spread about 0 and
+// x of one sign each is some 30 times what is left, and the error of a sum of x is
+// the same in every row.  In fp32 that left 9e-7 to 13e-7 of y (the VALU form, which
+// cancels them per 32 columns, 5e-7 to 6e-7); fp64 costs 3-4 % of a call.  rms error
+// against 64 bits over 2048 rows, in 1e-7 of the rms of y, here and in the VALU
+// form, for two kinds of weights and 2048 to 8192 columns: normal x 0.5-0.7
+// (1.0-2.6), one value per super-block 100 to 30000 times the others 0.5-0.7
+// (1.1-2.5), log-normal magnitudes with sigma 3 0.5-0.6 (0.9-1.9), all x positive
+// 0.4-0.6 (0.4-5.8).
 //
 // Q6_K the same way: the codes enter as signed bytes 4 (q - 32) (the high two
 // bits stored with 32's flipped, so that two masks and an or make four), each
 // MFMA's lane groups hold one 16-value sub-block each, so a lane (p, c) receives
 // digit p's sums of row c over four of them and weighs them by their signed
-// scales (below 2^29 together).  There are no minima.  rms error as above: normal
-// x 0.7e-7 to 0.9e-7 (1.5e-7 to 2.0e-7), outliers 0.8e-7 to 0.9e-7 (1.1e-7 to
-// 1.3e-7), log-normal 0.7e-7 to 0.9e-7 (1.3e-7), all positive 0.7e-7 (1.1e-7 to
-// 1.7e-7).
+// scales (below 2^29 together).  There are no minima, and fp32 sums do.  rms
+// error as above: normal x 0.6-0.7 (1.5-2.0), outliers 0.6-0.7 (1.1-1.9), log-normal
+// 0.6-0.7 (1.3-1.9), all positive 0.5-0.7 (1.1-2.6).
 //
 // Q8_0's codes are the B operand's bytes as they are; a lane (p, c) receives the
 // sums over blocks 2 g and 2 g + 1 as with Q4_K, below 2^20 and so exact in
-// fp32, where the blocks' fp16 scales meet them.  rms
-// error: normal x 0.9e-7 to 1.0e-7 (1.3e-7), outliers 0.6e-7 to 0.9e-7 (1.4e-7 to
-// 1.6e-7), log-normal 0.7e-7 to 0.9e-7 (1.2e-7 to 1.4e-7), all positive 0.8e-7 to
-// 1.0e-7 (1.2e-7).
+// fp32, where the blocks' fp16 scales meet them.  rms error: normal x 0.8-0.9
+// (1.3), outliers 0.6-0.8 (1.4-1.5), log-normal 0.6-0.7 (0.8-1.4), all positive 0.8
+// (1.1-1.3).
 //
 // Work split: a workgroup of NW waves takes RT tiles of 16 rows; wave v takes
 // super-blocks [v NSB, (v + 1) NSB) of all of them, whose x' it prepares for
@@ -534,6 +535,17 @@ __device__ __forceinline__ float rows_sum(float v) {
     v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
     auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+template <int CTRL> __device__ __forceinline__ double dpp(double v) {
+    return __hiloint2double((int)dpp<CTRL>((uint32_t)__double2hiint(v)), (int)dpp<CTRL>((uint32_t)__double2loint(v)));
+}
+__device__ __forceinline__ double rows_sum(double v) {
+    auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+    auto l = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+    v = __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+    h = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+    l = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
 }
 __device__ __forceinline__ uint32_t rows_max(uint32_t v) {
     auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
@@ -673,7 +685,8 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
     __builtin_amdgcn_sched_barrier(0);
 
     if (lane < 16) *(uint32_t *)(s_zero[wave] + 4 * lane) = 0;
-    float S0[NSB], S1[NSB], wgt[NSB], ss = 0.f;
+    double S0[NSB], S1[NSB];
+    float wgt[NSB], ss = 0.f;
     uint32_t plain = 0;
 #pragma unroll
     for (int s = 0; s < NSB; s++) {
@@ -689,11 +702,11 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
             for (int e = 0; e < 4; e++) v[e] = v[e] / (1.f + expf(-v[e])) * g[e];
         }
         if constexpr (!Q6 && !Q8) {  // sums over the sub-blocks (8 lanes) of this lane group: 2 grp, 2 grp + 1
-            float a = (v[0] + v[1]) + (v[2] + v[3]);
+            double a = ((double)v[0] + v[1]) + ((double)v[2] + v[3]);
             a += dpp<0xB1>(a);
             a += dpp<0x4E>(a);
             a += dpp<0x141>(a);
-            const float b = dpp<0x128>(a);  // the other 8 lanes of the row
+            const double b = dpp<0x128>(a);  // the other 8 lanes of the row
             S0[s] = (lane & 8) ? b : a;
             S1[s] = (lane & 8) ? a : b;
         }
@@ -721,9 +734,10 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
             const float r = (u - (float)t[0][j]) * 1073741824.f;
             t[1][j] = (int)r;
             left |= r != (float)t[1][j];
-            if (e > 156) left |= u == 0.f && v[j] != 0.f;  // s is below 1: the product underflowed
         }
-        if (__ballot(left)) {  // no digits: plain_dot takes the super-block
+        // no digits (with s below 1, e > 156, the product may underflow as
+        // well): plain_dot takes the super-block
+        if (__ballot(left) != 0 || e > 156) {
             plain |= 1u << s;
             wgt[s] = S0[s] = S1[s] = 0.f;
             *(float4 *)(s_x[wave][s][0] + 16 * lane) = make_float4(v[0], v[1], v[2], v[3]);
@@ -747,7 +761,9 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
         }
     }
     wave_order();
-    float acc[RT] = {};
+    // Q4_K's products and minima cancel: fp64 until they have
+    using Sum = std::conditional_t<Q6 || Q8, float, double>;
+    Sum acc[RT] = {};
     // row c of the A operand: digit c / 4 in the columns of group c % 4
     const int zoff = (c & 3) == grp ? grp * 256 + (c >> 2) * 64 : -1;
 #pragma unroll
@@ -827,8 +843,9 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
             const float d = h2f(dd[i][s] & 0xFFFF), dmin = h2f(dd[i][s] >> 16);
             const uint32_t kg = grp & 2 ? (grp & 1 ? k[3] : k[2]) : (grp & 1 ? k[1] : k[0]);
             const float m0 = (float)((kg >> 16) & 0xFFu), m1 = (float)(kg >> 24);
-            acc[i] = fmaf(d, fmaf((float)t[1], 0x1p-30f, (float)t[0]) * wgt[s], acc[i]);
-            acc[i] = fmaf(-dmin, fmaf(m0, S0[s], m1 * S1[s]), acc[i]);
+            acc[i] = fma((double)(-dmin * m0), S0[s], acc[i]);
+            acc[i] = fma((double)(-dmin * m1), S1[s], acc[i]);
+            acc[i] = fma((double)(d * wgt[s]), fma((double)t[1], 0x1p-30, (double)t[0]), acc[i]);
         }
     }
     if (plain) {
@@ -845,7 +862,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
     }
 #pragma unroll
     for (int i = 0; i < RT; i++) {
-        const float r = rows_sum(acc[i]);  // the digits' and the groups' shares of row c
+        const float r = (float)rows_sum(acc[i]);  // the digits' and the groups' shares of row c
         if (grp == 0) s_p[wave][i][c] = r;
     }
     if constexpr (MODE == 1) {
@@ -862,11 +879,15 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
         for (int v = 0; v < NW; v++) t += s_ss[v];
         rr = 1.0f / sqrtf(t / (float)w.cols + eps);
     }
-    auto sum = [&](int i, int r) {
-        float t = 0.f;
+    auto sum = [&](int i, int r) {  // pairwise: half the roundings of a chain
+        float t[NW];
 #pragma unroll
-        for (int v = 0; v < NW; v++) t += s_p[v][i][r];
-        return MODE == 1 ? t * rr : t;
+        for (int v = 0; v < NW; v++) t[v] = s_p[v][i][r];
+#pragma unroll
+        for (int n = NW; n > 1; n = (n + 1) / 2)
+#pragma unroll
+            for (int v = 0; v < n / 2; v++) t[v] = t[v] + t[n - 1 - v];
+        return MODE == 1 ? t[0] * rr : t[0];
     };
     const int i = tid >> 4, r = tid & 15;
     if (out_swiglu) {

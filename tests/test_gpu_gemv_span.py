@@ -1,6 +1,6 @@
 """What the matrix-core GEMVs (hymt2sharp_amd/csrc/gemv.hip, gemv_kq_kernel) make
-of inputs whose values lie far apart: infinities and NaN, and values far below
-their super-block's largest, which lose nothing to it.
+of inputs whose values lie far apart: infinities and NaN, values far below
+their super-block's largest, which lose nothing to it, and sums that cancel.
 
 Bound of the finite ones, root mean square over the rows: 2e-7 of the root mean
 square of y, about 3.4 roundings of 2^-24.  fp32 products added in fp32 make
@@ -140,3 +140,22 @@ def test_tiny_values(hip_available, wtype, scale):
     y = gemv(wtype, raw, 512, 2048, x)
     assert np.any(y != 0)
     check(y, W @ x.astype(np.float64))
+
+
+@pytest.mark.parametrize("cols", [2048, 4096, 6144, 8192])
+def test_q4k_sums_that_cancel(hip_available, cols):
+    """Weights spread evenly about 0 (codes times 8 d less 60 d) and inputs all
+    of one sign: a row's products and its minima are each about 30 times what
+    is left, and both meet the same sums of x in every row.  fp32 leaves 5e-7
+    and more."""
+    rows = 512
+    rng = np.random.default_rng(cols)
+    b = rng.integers(0, 256, (rows, cols // 256, 144), dtype=np.uint8)
+    d = rng.uniform(0.001, 0.002, (rows, cols // 256)).astype(np.float16)
+    b[:, :, 0:2] = b[:, :, 2:4] = d[..., None].view(np.uint8)
+    b[:, :, 4:16] = [8] * 4 + [60 | 3 << 6] * 4 + [8 | 12 << 4] * 4  # 8 scales of 8, 8 minima of 60
+    raw = b.tobytes()
+    W = O.dequant(N.W_Q4_K, raw, rows, cols).astype(np.float64)
+    assert abs(W.mean()) < 0.01 * W.std()
+    x = np.abs(rng.standard_normal(cols)).astype(np.float32)
+    check(gemv(N.W_Q4_K, raw, rows, cols, x), W @ x.astype(np.float64))
