@@ -50,15 +50,6 @@ __device__ __forceinline__ void bytes4(uint32_t w, float *o) {
     o[3] = (float)(w >> 24);
 }
 
-// w & mask with the mask hidden from the optimiser: bytes4 of the result is
-// then one v_cvt_f32_ubyteN per byte, where a visible mask would be folded
-// into a bit-field extract per byte before each conversion
-__device__ __forceinline__ uint32_t masked(uint32_t w, uint32_t mask) {
-    uint32_t r = w & mask;
-    asm("" : "+v"(r));
-    return r;
-}
-
 // x is staged in LDS with 4 floats of padding after every 64, so that the
 // 16-byte reads of the lanes of a wave (every row of the wave reads the same
 // 8 or 16 addresses, 64 floats apart) fall in different banks
@@ -480,11 +471,11 @@ __global__ __launch_bounds__(256) void embed_kernel(WeightDev w, int row, float 
 //    four signed bytes each, sum_p d_p 256^p; s is the power of two that brings
 //    the super-block's largest |x'| to [2^29, 2^30).  That holds every fp32
 //    value down to 2^-36 of the largest exactly.  A super-block with smaller
-//    ones (but 0), an infinity or NaN takes fp32 products instead (plain_dot).
+//    ones (but 0), one above 2^30, an infinity or NaN takes fp32 products instead
+//    (plain_dot).
 //    h alone lost what lay 2^-30 below the largest: beside a value 3000 times
-//    the others, at weight 0, the error was 2.1e-6 (1.2e-7 with l); l costs a
-//    second set of products, 2-8 % of a call (three layers' worth of Q4_K GEMVs
-//    1 %, 120818 x 2048 25.3 -> 28.3 us; Q8_0 there 47.4 -> 44.5).
+//    the others, at weight 0, the error was 2.1e-6 (under 1e-7 with l); l costs
+//    a second set of products, 1-4 % of eight layers' GEMVs;
 //  - the A operand's 16 rows are (digit p, sub-block pair g): row 4 p + g holds
 //    digit p of h (or l) in the k range of lane group g and zeros elsewhere, its 16
 //    columns are weight rows.  So a lane (p, c) receives digit p's sums of row
@@ -623,10 +614,10 @@ template <int T> __device__ __forceinline__ float plain_dot(const uint8_t *tile,
 }
 
 template <int T, int RT, int NW, int NSB, int MODE>
-__global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const float *__restrict__ xg,
+__global__ __launch_bounds__(64 * NW, T == kW_Q6_K && RT == 2 && NW == 8 && NSB == 1 ? 6 : 1) void gemv_kq_kernel(WeightDev w, const float *__restrict__ xg,
                                                           float *__restrict__ y, int flags,
                                                           const float *__restrict__ nw, float eps) {
-    constexpr bool Q6 = T == kW_Q6_K, Q8 = T == kW_Q8_0;
+    constexpr bool Q6 = T == kW_Q6_K, Q8 = T == kW_Q8_0, kLean = RT == 2 && (Q6 || (!Q8 && NW * NSB > 8));
     constexpr int kTile = Q8 ? kQ8Tile : Q6 ? kQ6Tile : kQ4Tile;
     // a wave's super-blocks as digits, [first, second][group][digit][64
     // columns], or as they are (the bits of `plain`), and zeros
@@ -768,13 +759,25 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
     const int zoff = (c & 3) == grp ? grp * 256 + (c >> 2) * 64 : -1;
 #pragma unroll
     for (int s = 0; s < NSB; s++) {
+        const i32x4 *xp[2];
+#pragma unroll
+        for (int d = 0; d < 2; d++) xp[d] = (const i32x4 *)(zoff < 0 ? s_zero[wave] : s_x[wave][s][d] + zoff);
         i32x4 xa[2][4];  // Q4_K: low codes' columns, high codes'
+        if constexpr (!kLean) {
 #pragma unroll
-        for (int d = 0; d < 2; d++) {
-            const i32x4 *xp = (const i32x4 *)(zoff < 0 ? s_zero[wave] : s_x[wave][s][d] + zoff);
+            for (int d = 0; d < 2; d++)
 #pragma unroll
-            for (int m = 0; m < 4; m++) xa[d][m] = xp[m];
+                for (int m = 0; m < 4; m++) xa[d][m] = xp[d][m];
         }
+        // Two tiles (kLean): xa's pieces read again for each tile, none moved
+        // ahead of the products before, instead of 32 registers held over both.
+        // Q6_K then fits six waves on a SIMD: 120818 x 2048 38.0 -> 36.1 us (Q8_0
+        // does not gain, 44.5 / 45.3, nor Q4_K with 8 super-blocks, whose 12288 x
+        // 2048 + SwiGLU takes 6.17 instead of 6.00; with more it saves spills).
+        auto again = [&](int d, int m) {
+            asm volatile("" ::: "memory");
+            xa[d][m] = xp[d][m];
+        };
 #pragma unroll
         for (int i = 0; i < RT; i++) {
             const uint4 a = q0[i][s], b = q1[i][s];
@@ -807,6 +810,11 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
                 int t[2] = {0, 0};
 #pragma unroll
                 for (int m = 0; m < 4; m++) {  // columns 64 g + 16 m + [0, 16): sub-block 4 g + m
+                    if constexpr (kLean) {
+                        if (m % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+                        again(0, m);
+                        again(1, m);
+                    }
                     i32x4 f;
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
@@ -831,6 +839,11 @@ __global__ __launch_bounds__(64 * NW) void gemv_kq_kernel(WeightDev w, const flo
             int t[2] = {0, 0};
 #pragma unroll
             for (int d = 0; d < 2; d++) {
+                if constexpr (kLean) {
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int m = 0; m < 4; m++) again(d, m);
+                }
                 i32x4 L = {0, 0, 0, 0}, H = {0, 0, 0, 0};
                 L = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[d][0], l0, L, 0, 0, 0);
                 H = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[d][2], h0, H, 0, 0, 0);
@@ -1070,24 +1083,24 @@ void launch_kq_mode(const WeightDev &w, const float *x, float *y, int flags, con
 // One tile per workgroup (with SwiGLU a gate and an up tile) and k over as many
 // waves as leave each one or two super-blocks, while that is at most 512
 // workgroups; beyond, 8 waves and two tiles that share a preparation of x'
-// (one at 8192 columns, where two would hold 140 registers).  us per call in a
+// (one at 8192 columns, where two would hold 200 registers).  us per call in a
 // recorded chain, W from HBM, the VALU form / here: 3072 x 2048 + norm 3.7 /
-// 3.3, 2048 x 2048 3.35 / 3.05, 12288 x 2048 + norm + SwiGLU 7.4 / 5.9, 2048 x
-// 6144 5.2 / 4.9 (12 waves of two super-blocks; 8 of three 5.0), 2048 x 8192 in
-// 16 waves 5.5, in 8 6.0; with the norm, 8192 x 2048 4.6 (two tiles 4.6), 16384
-// x 2048 9.1 / 6.2 (one tile 6.4), 40000 x 2048 26 / 11.3, 120818 x 2048 74 /
-// 26.5 (one tile 31.4, four 28.1).
+// 3.3, 2048 x 2048 3.05 / 2.9, 12288 x 2048 + norm + SwiGLU 6.8 / 6.0, 2048 x
+// 6144 4.7 / 4.75 in 12 waves of two super-blocks, 2048 x 8192 5.6 / 5.6 in 16;
+// with the norm 16384 x 2048 8.6 / 6.3, 40000 x 2048 25.5 / 12.4, 120818 x 2048
+// 72.5 / 29.3.
 // Q6_K by the same rule, the VALU form / here: 3072 x 2048 + norm 4.0 / 3.5, 2048 x
-// 2048 3.25 / 2.9, 12288 x 2048 + norm + SwiGLU 8.5 / 6.8, 2048 x 6144 5.9 / 4.8,
-// 2048 x 8192 7.1 / 5.5, with the norm 16384 x 2048 10.2 / 7.4, 40000 x 2048
-// 17.8 / 13.6, 120818 x 2048 42.5 / 36.4 (5.6 TB/s).
+// 2048 3.2 / 2.95, 12288 x 2048 + norm + SwiGLU 8.4 / 7.1, 2048 x 6144 5.9 / 5.3,
+// 2048 x 8192 7.2 / 6.2, with the norm 16384 x 2048 10.3 / 7.6, 40000 x 2048
+// 17.7 / 14.0, 120818 x 2048 42 / 36.1 (5.65 TB/s).
 // Q8_0 likewise (its VALU form had a byte convert and an fma per weight and fp32
-// scales): 4.0 / 3.7, 3.1 / 2.7, 7.3 / 7.1, 5.7 / 4.8, 6.9 / 5.8, 9.4 / 8.4, 18.1 /
-// 17.8, 47.5 / 46.5 (5.65 TB/s).  With SwiGLU Q8_0 takes tiles of 8 gate and 8 up
+// scales): 3.95 / 3.6, 3.1 / 2.9, 7.3 / 7.15, 5.7 / 5.1, 6.9 / 6.1, 9.4 / 8.5, 18.0 /
+// 16.7, 48.3 / 44.9 (5.85 TB/s).  With SwiGLU Q8_0 takes tiles of 8 gate and 8 up
 // rows, twice the workgroups (768 rather than 384 for 12288 rows, three per CU):
 // half a tile's codes are whole 128-byte lines, as its 4352 bytes are 34 lines.
-// One token through eight layers 164.0 -> 160.0 us; the other types' tiles start
-// within a line, and halves cost them (Q6_K 161.6 -> 169.5, Q4_K 149.1 -> 151.3).
+// One token through eight layers 164.0 -> 160.0 us when that was measured; the
+// other types' tiles start within a line, and halves cost them (Q6_K 161.6 ->
+// 169.5, Q4_K 149.1 -> 151.3).
 template <int T>
 hipError_t launch_kq(const WeightDev &w, const float *x, float *y, int flags, const float *nw, float eps,
                      hipStream_t s) {
