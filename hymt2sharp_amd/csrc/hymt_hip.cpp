@@ -1032,15 +1032,21 @@ struct hymt_weight {
     uint16_t *dense = nullptr;  // bf16 [rows][cols] copy for the prefill GEMMs (hymt_weight_dense)
 };
 
-// A Q4_K, Q6_K or Q8_0 matrix into its tiles, through a device buffer of at most 32 MiB that
-// the call owns (a few rows of tiles at a time), on the null stream as the
-// other types' copy.  Rearranged on the host, the 61-row layer's weights
+// A Q4_K, Q6_K or Q8_0 matrix into its tiles, through a device buffer of at
+// most 32 MiB that the call owns (a few rows of tiles at a time; less where the
+// device has no room, down to one row of tiles, 140 KB), on the null stream as
+// the other types' copy.  Rearranged on the host, the 61-row layer's weights
 // (36 MiB) took 7 ms longer to upload.
 static hipError_t upload_kq(int type, int rows, int cols, const uint8_t *data, uint8_t *mem) {
     const size_t rb = (size_t)hymt::gguf_row_bytes(type, cols);
-    const int step = (int)std::min<size_t>((32u << 20) / rb / 16 * 16, ((size_t)rows + 15) / 16 * 16);
+    int step = (int)std::min<size_t>((32u << 20) / rb / 16 * 16, ((size_t)rows + 15) / 16 * 16);
     uint8_t *tmp = nullptr;
     hipError_t e = hipMalloc((void **)&tmp, rb * (size_t)std::min(step, rows));
+    while (e == hipErrorOutOfMemory && step > 16) {
+        (void)hipGetLastError();
+        step = std::max(16, step / 32 * 16);
+        e = hipMalloc((void **)&tmp, rb * (size_t)std::min(step, rows));
+    }
     if (e != hipSuccess) return e;
     for (int r = 0; r < rows && e == hipSuccess; r += std::min(step, rows - r)) {
         const int n = std::min(step, rows - r);
