@@ -1251,8 +1251,8 @@ int hymt_gemm_swiglu(hymt_ctx *c, const hymt_weight *gate, const hymt_weight *up
         if (!gemm_swiglu(c->gemm, c->stream, gate->dense, wu, up != nullptr, f, k, (const uint16_t *)x, m, nullptr,
                          (uint16_t *)act, false, e))
             return fail(HYMT_E_UNSUPPORTED,
-                        "no fused gate/up + SwiGLU with the unfused calls' bits here (the GEMM mode, a k split for "
-                        "this prompt length, the shape or a misaligned x / act)");
+                        "no fused gate/up + SwiGLU here (the GEMM mode, a prompt so short that the 128-wide tiles' "
+                        "plan splits k, the shape or a misaligned x / act)");
         HIP_TRY(e);
     } catch (const HipError &e) {
         return map_hip(e);

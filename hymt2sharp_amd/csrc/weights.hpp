@@ -149,11 +149,13 @@ hipError_t gemm_swiglu_mfma(const uint16_t *Wg, const uint16_t *Wu, int f, int k
 // The state's fused gate/up + SwiGLU: runs it and returns true when the
 // state's choice for the unfused calls -- the gate/up GEMM(s) into gu (bf16
 // [m][2 f], as one [gate; up] matrix, or, separate, two [f][k] matrices) and
-// launch_rows_swiglu_bf16 -- is the MFMA kernel unsplit for every GEMM and the
-// 16-byte row kernel, so that the fused call's bits equal theirs; else returns
-// false having enqueued nothing (the caller issues the unfused calls).
-// With short_too it also serves prompts whose unfused GEMMs split k in the
-// short-prompt kernel (the fused form keeps their bits; hymt_gemm_swiglu
+// launch_rows_swiglu_bf16 -- is this library's MFMA kernels and the 16-byte row
+// kernel, and gemm_mfma.hip's plan for each GEMM does not split k (also where the
+// short-prompt kernel serves in its place), so that the fused call's bits equal
+// theirs; else returns false having enqueued nothing (the caller issues the
+// unfused calls).
+// With short_too it also serves the lengths that plan would split and the
+// short-prompt kernel takes (its fused form keeps its bits; hymt_gemm_swiglu
 // refuses those lengths, the model's prefill takes them).
 bool gemm_swiglu(GemmState *g, hipStream_t s, const uint16_t *Wg, const uint16_t *Wu, bool separate, int f, int k,
                  const uint16_t *x, int m, const uint16_t *gu, uint16_t *act, bool short_too, hipError_t &err);

@@ -379,10 +379,14 @@ int hymt_to_bf16(hymt_ctx *ctx, const float *x, size_t count, void *out);
  * one weight of 2 f rows [gate; up] with up NULL, or the f gate rows with up
  * the f up rows.  It runs only where its bits equal those of hymt_gemm with
  * HYMT_GEMM_OUT_BF16 into a bf16 [m][2 f] buffer (the two halves by two calls
- * for two weights) followed by hymt_rows_swiglu_bf16: the context's GEMM
- * choice is the hand-written MFMA kernel, unsplit, for those calls, f a
- * multiple of 64, cols a multiple of 128; otherwise it returns
- * HYMT_E_UNSUPPORTED and enqueues nothing, and the caller issues those calls.
+ * for two weights) followed by hymt_rows_swiglu_bf16, and not at the shortest
+ * prompts: the context's GEMM choice for those calls is the hand-written MFMA
+ * kernels, the 128-wide one's plan for the length does not split k (a length
+ * that it would split is refused whether or not the short-prompt kernel, which
+ * has a fused form with the same bits, would take it: 12288 gate/up rows run
+ * from 65 prompt rows on), f is a multiple of 64 and cols of 128; otherwise it
+ * returns HYMT_E_UNSUPPORTED and enqueues nothing, and the caller issues those
+ * calls.
  * x, act device pointers, 16-byte aligned; not recordable. */
 int hymt_gemm_swiglu(hymt_ctx *ctx, const hymt_weight *gate, const hymt_weight *up, const void *x, int m,
                      void *act);
