@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 
 from hymt2sharp_amd import HipBackend
-from hymt2sharp_amd._native import BF16, F16, F32
+from hymt2sharp_amd import synth as S
+from hymt2sharp_amd._native import BF16, F16, F32, ArgumentError
 from tests.attn_cases import BASE, D, EPS, HKV, HQ, cache_rows, max_rel, new_token
 from tests.test_gpu_random_sweep import decode_case
 from tests.test_gpu_decode import ulp_close
@@ -22,6 +23,52 @@ def test_short_cache(oracle, hip_available, dtype, pos):
     got, ref, (kd, vd), (kr, vr) = decode_case(oracle, dtype, pos, "gamma", config=17, salt=pos)
     assert max_rel(got, ref) <= 1e-3
     assert ulp_close(kd, kr, dtype) and ulp_close(vd, vr, dtype)
+
+
+@pytest.mark.parametrize("dtype,last", [(F32, 192), (F16, 512), (BF16, 512)])
+def test_one_launch_up_to(hip_available, dtype, last):
+    """No merge follows up to `last` cached positions; one does from the next."""
+    q, k, v, qnw, knw = new_token(17, 9, "gamma")
+    be = HipBackend(0).configure(HQ, HKV, D, D, BASE, EPS).create_cache(1, 640, dtype)
+    try:
+        be.MapRange(0, 640)
+        ptrs = dev_inputs(be, [q, k, v, qnw, knw])
+        out = be.alloc(q.nbytes)
+        be.timing_enable(2)
+        for n, pos in enumerate((1, 64, 65, 130, last), 1):
+            be.decode_dev(0, pos, *ptrs, out)
+            be.sync()
+            assert be.timing("decode_attn")[0] == n
+        with pytest.raises(ArgumentError):  # none was timed
+            be.timing("decode_merge")
+        be.decode_dev(0, last + 1, *ptrs, out)
+        be.sync()
+        assert be.timing("decode_merge")[0] == 1
+    finally:
+        be.Dispose()
+
+
+@pytest.mark.parametrize("kv_heads", [1, 2, 8])
+@pytest.mark.parametrize("dtype,pos", [(F32, 190), (F16, 100), (BF16, 400)])
+def test_other_kv_head_counts(oracle, hip_available, dtype, pos, kv_heads):
+    """The first kv heads of the usual inputs, or those twice over."""
+    def cut(a, per):  # per: heads for each kv head
+        return np.ascontiguousarray(np.concatenate([a, a], 1)[:, :per * kv_heads * D])
+    kb, vb = (cut(a, 1) for a in cache_rows(19, pos))
+    q, k, v, qnw, knw = new_token(19, 0, "gamma")
+    q, k, v = cut(q, 4), cut(k, 1), cut(v, 1)
+    be = HipBackend(0).configure(4 * kv_heads, kv_heads, D, D, BASE, EPS).create_cache(1, 640, dtype)
+    try:
+        be.UploadKv(0, 0, pos, kb, vb)
+        got = be.DecodeAttention(0, pos, q[0], k[0], v[0], qnw, knw)
+    finally:
+        be.Dispose()
+    caches = []
+    for b in (kb, vb):
+        caches.append(oracle.new_cache(640, kv_heads, D, dtype))
+        caches[-1][:pos] = oracle.to_storage(S.bf16_bits_to_f32(b), dtype)
+    ref = oracle.decode_attention(q[0], k[0], v[0], qnw, knw, *caches, dtype, 4 * kv_heads, kv_heads, D, BASE, EPS, pos)
+    assert max_rel(got, ref) <= 1e-3
 
 
 @pytest.mark.parametrize("dtype,rope_dim", [(F16, 64), (BF16, 2), (F32, 0)])

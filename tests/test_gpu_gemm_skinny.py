@@ -18,33 +18,57 @@ def default_choice(monkeypatch):
     monkeypatch.delenv("HYMT_HIP_GEMM_TILE", raising=False)
 
 
-@pytest.mark.parametrize("rows,cols,m", [
-    (128, 2048, 1), (2048, 2048, 16),                      # 16 x 16
-    (128, 2048, 17), (2048, 6144, 33), (2048, 8192, 64),   # 16 x 32 once 16 x 16 passes 256 workgroups
-    (12288, 2048, 1), (12288, 2048, 16),                   # 48 x 16
-    (3072, 2048, 33), (2048, 2048, 128),                   # 32 x 32
-    (12288, 2048, 17), (3072, 2048, 128),                  # 48 x 32
-    (2048, 6144, 129), (2048, 2048, 256),                  # 32 x 64
-    (12288, 2048, 64), (3072, 4096, 256),                  # 48 x 64
-    (2048, 2048, 257), (2048, 6144, 448),                  # 64 x 64
-    (12288, 2048, 65), (3072, 2048, 511),                  # 96 x 64
-    (2048, 2048, 513), (2048, 6144, 768),                  # 64 x 96, its last token count
-    (2048, 2048, 769),                                     # past it: the 128-wide tiles
+# features x tokens of the family's tiles, smallest first, in blocks of 16
+TILES = [(1, 1), (1, 2), (3, 1), (2, 2), (3, 2), (2, 4), (3, 4), (4, 4), (6, 4), (4, 6)]
+
+
+def tile(rows, m):
+    """The first tile that makes at most one round of 256 workgroups."""
+    for a, b in TILES:
+        if rows % (16 * a) == 0 and rows // (16 * a) * -(-m // (16 * b)) <= 256:
+            return a, b
+    return None
+
+
+@pytest.mark.parametrize("rows,cols,m,want", [
+    (128, 2048, 1, (1, 1)), (2048, 2048, 16, (1, 1)), (128, 2048, 17, (1, 1)),
+    (2048, 6144, 33, (1, 2)), (2048, 8192, 64, (1, 2)),
+    (12288, 2048, 1, (3, 1)), (12288, 2048, 16, (3, 1)), (3072, 2048, 33, (3, 1)),
+    (2048, 2048, 65, (2, 2)), (2048, 2048, 128, (2, 2)),
+    (12288, 2048, 17, (3, 2)), (3072, 2048, 128, (3, 2)),
+    (2048, 6144, 129, (2, 4)), (2048, 2048, 256, (2, 4)),
+    (12288, 2048, 64, (3, 4)), (3072, 4096, 256, (3, 4)),
+    (2048, 2048, 257, (4, 4)), (2048, 6144, 448, (4, 4)),
+    (12288, 2048, 65, (6, 4)), (3072, 2048, 511, (6, 4)),
+    (2048, 2048, 513, (4, 6)), (2048, 6144, 768, (4, 6)),  # its last token count
+    (2048, 2048, 769, None),                               # past it: the 128-wide tiles
 ])
-def test_tiles_and_edges(hip_available, rows, cols, m):
+def test_tiles_and_edges(hip_available, monkeypatch, rows, cols, m, want):
+    assert tile(rows, m) == want
     out, counts, ref, mag, y0 = run_case(rows, cols, m, 6000 + rows + cols + m, MFMA)
     check(out, ref, mag, y0)
     assert counts == {"gemm_mfma_out_f32": 2, "gemm_mfma_out_bf16": 1}
+    # which kernel it was: k in four parts here, whole in an unsplit tile of the
+    # other, whose tiles all give the same bits
+    monkeypatch.setenv("HYMT_HIP_GEMM_TILE", "128x64")
+    other, _, _, _, _ = run_case(rows, cols, m, 6000 + rows + cols + m, MFMA)
+    assert np.array_equal(out["f32"], other["f32"]) == (want is None)
 
 
-def test_bits_do_not_depend_on_the_tile(hip_available):
-    """The rows of a prompt give the same bits alone (a smaller tile) and as
+@pytest.mark.parametrize("rows,lengths", [(2048, [33, 100, 200, 400, 700]), (3072, [20, 50, 100, 200, 300, 500])])
+def test_bits_do_not_depend_on_the_tile(hip_available, rows, lengths):
+    """The rows of a prompt give the same bits alone (the smallest tile) and as
     part of a longer one: k is split the same way in every tile."""
-    whole, _, _, _, _ = run_case(256, 2048, 1, 11, MFMA)
-    for m in (17, 100, 400):  # run_case draws x row by row from the seed: row 0 is the same
-        part, _, _, _, _ = run_case(256, 2048, m, 11, MFMA)
+    whole, _, _, _, _ = run_case(rows, 2048, 1, 11, MFMA)
+    for m in lengths:  # run_case draws x row by row from the seed: row 0 is the same
+        part, _, _, _, _ = run_case(rows, 2048, m, 11, MFMA)
         assert np.array_equal(part["f32"][:1], whole["f32"]), m
         assert np.array_equal(part["bf16"][:1], whole["bf16"]), m
+
+
+def test_every_tile_is_compared():
+    seen = {tile(2048, m) for m in (1, 33, 100, 200, 400, 700)} | {tile(3072, m) for m in (20, 50, 100, 200, 300, 500)}
+    assert seen == set(TILES)
 
 
 @pytest.mark.parametrize("f,k,m,separate", [

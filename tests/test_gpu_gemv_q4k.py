@@ -4,12 +4,11 @@ one or two 16-row tiles a workgroup), row counts that do not fill a tile,
 the input and output modes, and inputs of extreme range, against the fp64
 product of the dequantized weights.
 
-Bound: x' is exact to 2^-30 of its super-block's largest value and the
-products are summed in integers, so what remains is fp32: one rounding per
-super-block and digit, the minima (8 fp32 sums of 32 values each) and the sum
-over cols / 256 super-blocks -- under 16 roundings of 2^-24 on terms that add up
-to sum |w x| + sum |min x|.  The minima exceed |w x| several times over for
-these random blocks; 4e-6 of sum |w x| covers them."""
+Bound: x' enters exactly, the products are summed in integers and with the
+minima in fp64; what remains is fp32, a rounding of each wave's share of a row
+and their sum: under 16 roundings of 2^-24 on terms that add up to sum |w x|,
+1e-6 of it.  The norm's factor and the sigmoid, and super-blocks that take fp32
+products (values 2^36 apart), add a few more: 4e-6."""
 import numpy as np
 import pytest
 
@@ -45,7 +44,7 @@ def run(rows, cols, x, seed, y0=None, **kw):
 
 
 def close(y, ref, mag):
-    assert np.all(np.abs(y - ref) <= 4e-6 * mag + 1e-30), float(np.max(np.abs(y - ref) / (mag + 1e-30)))
+    assert np.all(np.abs(y - ref) <= 4e-6 * mag), float(np.max(np.abs(y - ref) / mag))
 
 
 @pytest.mark.parametrize("cols", [2048, 4096, 6144, 8192])
@@ -102,9 +101,6 @@ def test_range(hip_available, kind):
     x = x.astype(np.float64)
     if kind == "zero":
         assert np.all(y == 0)
-    elif kind == "outlier":  # values 2^-15 of the largest keep 2^-30 of it: 2^-15 of themselves at worst
-        big = np.repeat(np.abs(x).reshape(-1, 256).max(1), 256)
-        close(y, W @ x, np.abs(W) @ (np.abs(x) + big * 2.0 ** -12))
     else:
         close(y, W @ x, np.abs(W) @ np.abs(x))
 
