@@ -613,11 +613,11 @@ template <int T> __device__ __forceinline__ float plain_dot(const uint8_t *tile,
     return y;
 }
 
-template <int T, int RT, int NW, int NSB, int MODE>
-__global__ __launch_bounds__(64 * NW, T == kW_Q6_K && RT == 2 && NW == 8 && NSB == 1 ? 6 : 1) void gemv_kq_kernel(WeightDev w, const float *__restrict__ xg,
+template <int T, int RT, int NW, int NSB, int MODE, bool MANY>
+__global__ __launch_bounds__(64 * NW, T != kW_Q8_0 && MANY && RT == 2 && NSB == 1 ? 6 : 1) void gemv_kq_kernel(WeightDev w, const float *__restrict__ xg,
                                                           float *__restrict__ y, int flags,
                                                           const float *__restrict__ nw, float eps) {
-    constexpr bool Q6 = T == kW_Q6_K, Q8 = T == kW_Q8_0, kLean = RT == 2 && (Q6 || (!Q8 && NW * NSB > 8));
+    constexpr bool Q6 = T == kW_Q6_K, Q8 = T == kW_Q8_0, kLean = RT == 2 && !Q8 && (MANY || NW * NSB > 8);
     constexpr int kTile = Q8 ? kQ8Tile : Q6 ? kQ6Tile : kQ4Tile;
     // a wave's super-blocks as digits, [first, second][group][digit][64
     // columns], or as they are (the bits of `plain`), and zeros
@@ -771,9 +771,10 @@ __global__ __launch_bounds__(64 * NW, T == kW_Q6_K && RT == 2 && NW == 8 && NSB 
         }
         // Two tiles (kLean): xa's pieces read again for each tile, none moved
         // ahead of the products before, instead of 32 registers held over both.
-        // Q6_K then fits six waves on a SIMD: 120818 x 2048 38.0 -> 36.1 us (Q8_0
-        // does not gain, 44.5 / 45.3, nor Q4_K with 8 super-blocks, whose 12288 x
-        // 2048 + SwiGLU takes 6.17 instead of 6.00; with more it saves spills).
+        // Where the grid is long (MANY) six waves then fit a SIMD: 120818 x 2048
+        // of Q6_K 38.0 -> 35.9 us, of Q4_K 29.4 -> 28.3 (Q8_0 does not gain, 44.5 /
+        // 45.3, nor a short grid, Q4_K 12288 x 2048 + SwiGLU 6.17 / 6.00); with more
+        // than 8 super-blocks it saves spills.
         auto again = [&](int d, int m) {
             asm volatile("" ::: "memory");
             xa[d][m] = xp[d][m];
@@ -1071,13 +1072,13 @@ hipError_t launch_t(const WeightDev &w, const float *x, float *y, int flags, con
     return hipGetLastError();
 }
 
-template <int T, int RT, int NW, int NSB>
+template <int T, int RT, int NW, int NSB, bool MANY>
 void launch_kq_mode(const WeightDev &w, const float *x, float *y, int flags, const float *nw, float eps, int grid,
                     const KernelSpan &span, hipStream_t s) {
     const dim3 g(grid), b(64 * NW);
-    if (flags & kGemvInRmsNorm) launch(span, gemv_kq_kernel<T, RT, NW, NSB, 1>, g, b, 0, s, w, x, y, flags, nw, eps);
-    else if (flags & kGemvInSwiGLU) launch(span, gemv_kq_kernel<T, RT, NW, NSB, 2>, g, b, 0, s, w, x, y, flags, nw, eps);
-    else launch(span, gemv_kq_kernel<T, RT, NW, NSB, 0>, g, b, 0, s, w, x, y, flags, nw, eps);
+    if (flags & kGemvInRmsNorm) launch(span, gemv_kq_kernel<T, RT, NW, NSB, 1, MANY>, g, b, 0, s, w, x, y, flags, nw, eps);
+    else if (flags & kGemvInSwiGLU) launch(span, gemv_kq_kernel<T, RT, NW, NSB, 2, MANY>, g, b, 0, s, w, x, y, flags, nw, eps);
+    else launch(span, gemv_kq_kernel<T, RT, NW, NSB, 0, MANY>, g, b, 0, s, w, x, y, flags, nw, eps);
 }
 
 // One tile per workgroup (with SwiGLU a gate and an up tile) and k over as many
@@ -1087,8 +1088,8 @@ void launch_kq_mode(const WeightDev &w, const float *x, float *y, int flags, con
 // recorded chain, W from HBM, the VALU form / here: 3072 x 2048 + norm 3.7 /
 // 3.3, 2048 x 2048 3.05 / 2.9, 12288 x 2048 + norm + SwiGLU 6.8 / 6.0, 2048 x
 // 6144 4.7 / 4.75 in 12 waves of two super-blocks, 2048 x 8192 5.6 / 5.6 in 16;
-// with the norm 16384 x 2048 8.6 / 6.3, 40000 x 2048 25.5 / 12.4, 120818 x 2048
-// 72.5 / 29.3.
+// with the norm 16384 x 2048 8.6 / 6.4, 40000 x 2048 25.5 / 11.7, 120818 x 2048
+// 72.5 / 28.3.
 // Q6_K by the same rule, the VALU form / here: 3072 x 2048 + norm 4.0 / 3.5, 2048 x
 // 2048 3.2 / 2.95, 12288 x 2048 + norm + SwiGLU 8.4 / 7.1, 2048 x 6144 5.9 / 5.3,
 // 2048 x 8192 7.2 / 6.2, with the norm 16384 x 2048 10.3 / 7.6, 40000 x 2048
@@ -1111,8 +1112,15 @@ hipError_t launch_kq(const WeightDev &w, const float *x, float *y, int flags, co
     KernelSpan span(gemv_span_name(w.type), s, true);
     auto go = [&](auto waves, auto sbs, int rt) {
         constexpr int NW = decltype(waves)::value, NSB = decltype(sbs)::value;
-        if (rt == 2) launch_kq_mode<T, 2, NW, NSB>(w, x, y, flags, nw, eps, (tiles + 1) / 2, span, s);
-        else launch_kq_mode<T, 1, NW, NSB>(w, x, y, flags, nw, eps, half ? (w.rows / 2 + 7) / 8 : tiles, span, s);
+        if (rt == 2) {  // 8 waves of several super-blocks each: long grids only
+            if (NW == 8 && (NSB > 1 || !few)) {
+                if constexpr (NW == 8) launch_kq_mode<T, 2, NW, NSB, true>(w, x, y, flags, nw, eps, (tiles + 1) / 2, span, s);
+            } else if constexpr (NW > 8 || NSB == 1) {
+                launch_kq_mode<T, 2, NW, NSB, false>(w, x, y, flags, nw, eps, (tiles + 1) / 2, span, s);
+            }
+        } else if constexpr (NW > 8 || NSB == 1 || NSB == 4) {
+            launch_kq_mode<T, 1, NW, NSB, false>(w, x, y, flags, nw, eps, half ? (w.rows / 2 + 7) / 8 : tiles, span, s);
+        }
     };
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
