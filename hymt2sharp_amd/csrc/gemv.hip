@@ -471,8 +471,8 @@ __global__ __launch_bounds__(256) void embed_kernel(WeightDev w, int row, float 
 //    four signed bytes each, sum_p d_p 256^p; s is the power of two that brings
 //    the super-block's largest |x'| to [2^29, 2^30).  That holds every fp32
 //    value down to 2^-36 of the largest exactly.  A super-block with smaller
-//    ones (but 0), one above 2^30, an infinity or NaN takes fp32 products instead
-//    (plain_dot).
+//    ones (but 0), one of 2^74, an infinity or NaN takes fp32 products instead
+//    (plain_dot), which take several times as long.
 //    h alone lost what lay 2^-30 below the largest: beside a value 3000 times
 //    the others, at weight 0, the error was 2.1e-6 (under 1e-7 with l); l costs
 //    a second set of products, 1-4 % of eight layers' GEMVs;
@@ -726,9 +726,11 @@ __global__ __launch_bounds__(64 * NW, T != kW_Q8_0 && MANY && RT == 2 && NSB == 
             t[1][j] = (int)r;
             left |= r != (float)t[1][j];
         }
-        // no digits (with s below 1, e > 156, the product may underflow as
-        // well): plain_dot takes the super-block
-        if (__ballot(left) != 0 || e > 156) {
+        // no digits: plain_dot takes the super-block.  So it does where the
+        // largest value is 2^74 or more, whose scale could take another to 0
+        // unnoticed; below that only values under 2^-105 beside one over 2^30
+        // are lost to it, which is 2^-135 of it
+        if (__ballot(left) != 0 || e > 200) {
             plain |= 1u << s;
             wgt[s] = S0[s] = S1[s] = 0.f;
             *(float4 *)(s_x[wave][s][0] + 16 * lane) = make_float4(v[0], v[1], v[2], v[3]);
