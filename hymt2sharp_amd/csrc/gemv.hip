@@ -551,66 +551,50 @@ __device__ __forceinline__ void wave_order() {
 }
 
 // Columns 64 grp + [0, 64) of a tile's row r times x, in fp32, a code and a
-// value at a time as the VALU form has them.  Loops, not registers: this is
-// the way of super-blocks whose x' has no digits.
+// value at a time as the VALU form has them: the way of super-blocks whose x'
+// has no digits.  16 columns at a time, so that the rare path takes no more
+// registers than the kernel around it.
 template <int T> __device__ __forceinline__ float plain_dot(const uint8_t *tile, int r, int grp, const float *x) {
-    const uint32_t *q = (const uint32_t *)(tile + 16 * (16 * grp + r));  // piece m's dword j: q[256 m + j]
+    const int at = 16 * (16 * grp + r);
     float y = 0.f;
-    if constexpr (T == kW_Q4_K) {  // sub-blocks 2 grp (low codes) and 2 grp + 1
-        const uint8_t *sm = tile + kQ4Scales + 16 * r + 4 * grp;
-        const uint32_t dd = *(const uint32_t *)(tile + kQ4D + 4 * r);
 #pragma unroll 1
-        for (int h = 0; h < 2; h++) {
-            float a = 0.f, sx = 0.f;
-#pragma unroll 1
-            for (int j = 0; j < 8; j++) {
-                const uint32_t k = q[256 * (j >> 2) + (j & 3)] >> (4 * h);
+    for (int m = 0; m < 4; m++) {  // columns 16 m + [0, 16)
+        const uint4 c4 = *(const uint4 *)(tile + 1024 * (T == kW_Q8_0 ? m : T == kW_Q6_K ? m >> 1 : m & 1) + at);
+        const uint32_t c[4] = {c4.x, c4.y, c4.z, c4.w};
+        uint4 h4 = make_uint4(0, 0, 0, 0);
+        if constexpr (T == kW_Q6_K) h4 = *(const uint4 *)(tile + kQ6Hi + at);
+        const uint32_t h[4] = {h4.x, h4.y, h4.z, h4.w};
+        float a = 0.f, sx = 0.f;
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float v = x[32 * h + 4 * j + e];
-                    a = fmaf((float)((k >> (8 * e)) & 0xFu), v, a);
-                    sx += v;
+        for (int j = 0; j < 4; j++) {
+            const float4 xv = *(const float4 *)(x + 16 * m + 4 * j);
+            const float v[4] = {xv.x, xv.y, xv.z, xv.w};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                if constexpr (T == kW_Q8_0) {
+                    a = fmaf((float)(int8_t)(c[j] >> (8 * e)), v[e], a);
+                } else if constexpr (T == kW_Q6_K) {  // the stored upper bit is flipped
+                    const uint32_t lo = c[j] >> (4 * (m & 1)), hb = h[j] >> (6 - 2 * m);
+                    a = fmaf((float)((int)(((lo >> (8 * e)) & 0xFu) | ((((hb >> (8 * e)) & 3u) ^ 2u) << 4)) - 32), v[e], a);
+                } else {
+                    a = fmaf((float)((c[j] >> (8 * e + 4 * (m >> 1))) & 0xFu), v[e], a);
                 }
+                sx += v[e];
             }
-            y += h2f(dd & 0xFFFF) * ((float)sm[h] * a) - h2f(dd >> 16) * ((float)sm[2 + h] * sx);
         }
-    } else if constexpr (T == kW_Q6_K) {  // sub-blocks 4 grp + m
-        const uint32_t *hi = (const uint32_t *)(tile + kQ6Hi + 16 * (16 * grp + r));
-        const int8_t *sc = (const int8_t *)(tile + kQ6Scales + 16 * r + 4 * grp);
-#pragma unroll 1
-        for (int m = 0; m < 4; m++) {
-            float a = 0.f, sx = 0.f;
-#pragma unroll 1
-            for (int j = 0; j < 4; j++) {
-                const uint32_t lo = q[256 * (m >> 1) + j] >> (4 * (m & 1)), hb = hi[j] >> (6 - 2 * m);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {  // the stored upper bit is flipped
-                    const uint32_t k = ((lo >> (8 * e)) & 0xFu) | ((((hb >> (8 * e)) & 3u) ^ 2u) << 4);
-                    const float v = x[16 * m + 4 * j + e];
-                    a = fmaf((float)(int)(k - 32u), v, a);
-                    sx += v;
-                }
-            }
+        if constexpr (T == kW_Q8_0) {
+            y += h2f(*(const uint16_t *)(tile + kQ8D + 16 * r + 4 * grp + 2 * (m >> 1))) * a;
+        } else if constexpr (T == kW_Q6_K) {
             // with the offset taken off afterwards (code v less 32 v) an
             // infinity of x' is NaN whatever the code: 0 sx keeps that
-            y += (float)sc[m] * fmaf(0.f, sx, a);
-        }
-        y *= h2f(*(const uint16_t *)(tile + kQ6D + 2 * r));
-    } else {  // blocks 2 grp, 2 grp + 1
-        const uint16_t *d = (const uint16_t *)(tile + kQ8D + 16 * r + 4 * grp);
-#pragma unroll 1
-        for (int h = 0; h < 2; h++) {
-            float a = 0.f;
-#pragma unroll 1
-            for (int j = 0; j < 8; j++) {
-                const uint32_t k = q[256 * (2 * h + (j >> 2)) + (j & 3)];
-#pragma unroll
-                for (int e = 0; e < 4; e++) a = fmaf((float)(int8_t)(k >> (8 * e)), x[32 * h + 4 * j + e], a);
-            }
-            y += h2f(d[h]) * a;
+            y += (float)*(const int8_t *)(tile + kQ6Scales + 16 * r + 4 * grp + m) * fmaf(0.f, sx, a);
+        } else {  // low codes, then high ones: sub-blocks 2 grp and 2 grp + 1
+            const uint8_t *sm = tile + kQ4Scales + 16 * r + 4 * grp + (m >> 1);
+            const uint32_t dd = *(const uint32_t *)(tile + kQ4D + 4 * r);
+            y += h2f(dd & 0xFFFF) * ((float)sm[0] * a) - h2f(dd >> 16) * ((float)sm[2] * sx);
         }
     }
-    return y;
+    return T == kW_Q6_K ? y * h2f(*(const uint16_t *)(tile + kQ6D + 2 * r)) : y;
 }
 
 template <int T, int RT, int NW, int NSB, int MODE, bool MANY>
