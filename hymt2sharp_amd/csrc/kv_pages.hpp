@@ -207,7 +207,8 @@ class KvPages {
     // These entries of the device table may not hold the table's values: they
     // are changed entries again.
     void mark_dirty(const std::vector<int> &entries) {
-        for (int b : entries) mark(b);
+        for (int b : entries)
+            if (b >= 0 && b < max_pages_) mark(b);
     }
     // The recording is closed, kept or not: what it would update is still to
     // do for every call that runs before it.  Returns those entries, which a

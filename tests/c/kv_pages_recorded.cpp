@@ -36,5 +36,9 @@ int main() {
     p.mark_dirty(kept);  // two replays
     CHECK((p.take_dirty() == Ints{5, 6}));
     CHECK(p.phys(5) == -1 && p.phys(6) == -1);
+
+    // entries of a larger context's recording are none of this table's
+    p.mark_dirty({-1, 10, 1000});
+    CHECK(!p.has_dirty());
     return 0;
 }
