@@ -162,10 +162,9 @@ int map_hip(const HipError &e) {
     return fail(HYMT_E_DEVICE, std::string(e.what) + ": " + hipGetErrorString(e.e));
 }
 
-// Mirror changed page-table entries to the device table.
-void flush_table(hymt_ctx *c) {
-    if (!c->pages.has_dirty()) return;
-    std::vector<int> idx = c->pages.take_dirty(c->capturing);
+// These entries of the page table to the device table.
+void write_table(hymt_ctx *c, const std::vector<int> &idx) {
+    if (idx.empty()) return;
     std::vector<int> val(idx.size());
     for (size_t i = 0; i < idx.size(); i++) val[i] = c->pages.phys(idx[i]);
     const hipError_t e = launch_tab_update((int32_t *)c->tab.p, idx.data(), val.data(), (int)idx.size(), c->stream);
@@ -173,6 +172,11 @@ void flush_table(hymt_ctx *c) {
         c->pages.mark_dirty(idx);
         HIP_TRY(e);
     }
+}
+
+// Mirror changed page-table entries to the device table.
+void flush_table(hymt_ctx *c) {
+    if (c->pages.has_dirty()) write_table(c, c->pages.take_dirty(c->capturing));
 }
 
 // Map [pos, pos+len) for writing: pages for unmapped blocks, fresh pages for
@@ -998,6 +1002,12 @@ int hymt_graph_launch(hymt_ctx *c, hymt_graph *g) {
                                   "reallocated (RoPE table or workspace growth); record it again");
     (void)hipSetDevice(c->device);
     TimedCall timed(call_timer(c), "graph_launch", 0);
+    // what another recording left to do, or its replay undid
+    try {
+        if (c->pages.has_dirty()) write_table(c, c->pages.take_mapped(g->tab));
+    } catch (const HipError &x) {
+        return map_hip(x);
+    }
     KernelSpan span("graph", c->stream);
     hipError_t e = hipGraphLaunch(g->exec, c->stream);
     c->pages.mark_dirty(g->tab);  // the table has moved on since the recording, perhaps

@@ -25,6 +25,7 @@
 // before launching kernels that read them.
 #pragma once
 
+#include <algorithm>
 #include <cstdint>
 #include <list>
 #include <stdexcept>
@@ -204,6 +205,17 @@ class KvPages {
         return d;
     }
     bool has_dirty() const { return !dirty_.empty(); }
+    // Of those, the ones that name a page and are not among `own`: what a
+    // recording that writes the entries `own` needs on the device beforehand.
+    // The others stay on the list.
+    std::vector<int> take_mapped(const std::vector<int> &own) {
+        std::vector<int> d, keep;
+        for (int b : dirty_)
+            (tab_[b] >= 0 && std::find(own.begin(), own.end(), b) == own.end() ? d : keep).push_back(b);
+        dirty_.assign(keep.begin(), keep.end());
+        for (int b : d) dirty_flag_[b] = 0;
+        return d;
+    }
     // These entries of the device table may not hold the table's values: they
     // are changed entries again.
     void mark_dirty(const std::vector<int> &entries) {

@@ -37,6 +37,15 @@ int main() {
     CHECK((p.take_dirty() == Ints{5, 6}));
     CHECK(p.phys(5) == -1 && p.phys(6) == -1);
 
+    // before another recording, which writes entry 5 itself, runs: the entries
+    // that name a page, and not its own
+    p.ensure_written(320, 192);  // 5, 6, 7
+    p.take_dirty();
+    p.mark_dirty({3, 5, 6});
+    p.set_len(385);  // 7 given back
+    CHECK((p.take_mapped({5}) == Ints{3, 6}));
+    CHECK((p.take_dirty() == Ints{5, 7}));
+
     // entries of a larger context's recording are none of this table's
     p.mark_dirty({-1, 10, 1000});
     CHECK(!p.has_dirty());

@@ -89,3 +89,56 @@ def test_replay_after_the_table_moved_on(hip_available):
         be.graph_destroy(g)
     finally:
         be.Dispose()
+
+
+@pytest.mark.gpu
+def test_replay_after_another_replay(hip_available):
+    """The page that one recording's replay writes into the device table is not
+    what the next one reads there."""
+    kb, vb = cache_rows(25, 320)
+    q, k, v, qnw, knw = new_token(25, 1, "gamma", seq=64)
+    be = HipBackend(0).configure(HQ, HKV, D, D, BASE, EPS).create_cache(1, 640, F16)
+    try:
+        be.UploadKv(0, 0, 256, kb, vb)
+        be.ReadKv(0, 0, 128)
+        ptrs = []
+        for a in (q, k, v, qnw, knw):
+            ptrs.append(be.alloc(a.nbytes))
+            be.upload(ptrs[-1], a)
+        out = be.alloc(q.nbytes)
+
+        def chunk():
+            be.prefill_dev(0, 256, 64, *ptrs[:3], F32, *ptrs[3:], out)
+
+        chunk()  # its workspace; maps page 4
+        be.SetCacheLen(256)
+        be.graph_begin()
+        be.decode_dev(0, 256, *ptrs, out)  # maps page 4
+        g1 = be.graph_end()
+        recorded = be.page_of(4)
+        be.SetCacheLen(192)
+        be.MapRange(192, 64)
+        be.UploadKv(0, 192, 64, kb, vb)
+        chunk()  # block 4 has another page
+        assert be.page_of(3) == recorded
+        be.graph_begin()
+        chunk()
+        g2 = be.graph_end()
+        want = be.ReadKv(0, 256, 64)
+        be.graph_launch(g1)          # a row of block 4 into block 3's page: undone by the upload
+        be.sync()
+        be.UploadKv(0, 192, 64, kb, vb)
+        three = be.ReadKv(0, 192, 64)
+        be.upload(ptrs[1], np.zeros_like(k))
+        be.upload(ptrs[2], np.zeros_like(v))
+        be.graph_launch(g1)
+        be.graph_launch(g2)          # block 4's own page, rows of 0
+        be.sync()
+        four = be.ReadKv(0, 256, 64)
+        assert not four[1].any() and want[1].any()
+        now = be.ReadKv(0, 192, 64)
+        assert np.array_equal(now[0][1:], three[0][1:]) and np.array_equal(now[1][1:], three[1][1:])
+        be.graph_destroy(g1)
+        be.graph_destroy(g2)
+    finally:
+        be.Dispose()
